@@ -31,6 +31,10 @@ __device__ __forceinline__ T gload(const T* p) {
     return *(const __attribute__((address_space(1))) T*)p;
 }
 
+// Four floats as the compiler's own vector type (HIP's float4 is a class, which
+// gload cannot read from global memory).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 // a / b for a divisor b shared by many quotients, from rb = RN64(1 / b):
 // RN32(RN64(a * rb)) is the IEEE binary32 quotient whenever that quotient is
 // a normal number.  Proof: the binary64 value is within 2^-52 (relative) of

@@ -243,14 +243,11 @@ constexpr uint32_t kInfBits = 0x7f800000u;  // +inf as float bits: unbounded dis
 // +inf when the node's weights could leave [e^-2, 1] (radius not positive or
 // 2r^2 outside the Markstein-safe range), its position or transform is not
 // finite, or the bound does not fit a float.
-__device__ uint32_t disp_bound_bits(const VolDesc& vd, const float* M, const float m[3], float r,
+__device__ uint32_t disp_bound_bits(const VolDesc& vd, const float e[16], const float m[3], float r,
                                     const int32_t vlo[3], const int32_t vhi[3]) {
     if (!(r > 0.0f) || !den_safe(2.0f * (r * r))) return kInfBits;
     if (!__builtin_isfinite(m[0]) || !__builtin_isfinite(m[1]) || !__builtin_isfinite(m[2])) return kInfBits;
-    float e[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) e[i] = M[i];  // column-major: M(a, j) = e[4 j + a]
-    bool fin = true;
+    bool fin = true;  // column-major: T(a, j) = e[4 j + a]
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
@@ -300,7 +297,7 @@ __device__ __forceinline__ float depth_key(float d) {
 __device__ void depth_tiles(const VolDesc* __restrict__ vols, int nvol, uint32_t blk, float* __restrict__ dmax) {
     __shared__ uint32_t s_pb[kMaxBatch];
     __shared__ float s_seg[kTile1][kTile1 / kTile0];
-    static_assert(kPrepThreads == kTile1 * (kTile1 / kTile0), "one thread per 16-pixel row segment");
+    static_assert(kTile0 == 16 && kTile1 * 32 % kPrepThreads == 0, "four lanes per 16-pixel row segment");
     const int tid = threadIdx.x;
     for (int v = tid; v < nvol; v += blockDim.x) s_pb[v] = vols[v].pyr_blk;
     __syncthreads();
@@ -316,17 +313,41 @@ __device__ void depth_tiles(const VolDesc* __restrict__ vols, int nvol, uint32_t
     const uint32_t local = blk - vd.pyr_blk;
     const int32_t bx = (int32_t)(local % (uint32_t)vd.pw1), by = (int32_t)(local / (uint32_t)vd.pw1);
     const int32_t W = vd.cam.W, H = vd.cam.H;
-    const int row = tid / (kTile1 / kTile0), seg = tid % (kTile1 / kTile0);
-    const int32_t y = by * kTile1 + row;
-    const int32_t x0 = bx * kTile1 + seg * kTile0;
-    float m = -kInf;
-    if (y < H) {
-        const float* rowp = vd.depth + (int64_t)y * W;
+    // 32 threads a row, four pixels each, four rows a thread: a wave reads two
+    // whole 512 B row spans.  Every load is issued before the first is used
+    // (places past the frame read its last pixels and count as -inf): with a
+    // branch around each load the thread waited for its 16 pixels one by one.
+    const int q = tid & 31, r0 = tid >> 5;
+    constexpr int kRows = kTile1 * 32 / kPrepThreads;
+    const int32_t x = bx * kTile1 + 4 * q;
+    float px[kRows][4];
+    if ((W & 3) == 0 && ((uintptr_t)vd.depth & 15u) == 0) {
+        const int32_t xc = x < W ? x : W - 4;
 #pragma unroll
-        for (int i = 0; i < kTile0; ++i)
-            if (x0 + i < W) m = fmaxf(m, depth_key(gload(rowp + x0 + i)));
+        for (int i = 0; i < kRows; ++i) {
+            const int32_t y = by * kTile1 + r0 + 32 * i;
+            const f32x4 v4 = gload((const f32x4*)(vd.depth + (int64_t)(y < H ? y : H - 1) * W + xc));
+            px[i][0] = v4.x, px[i][1] = v4.y, px[i][2] = v4.z, px[i][3] = v4.w;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            const int32_t y = by * kTile1 + r0 + 32 * i;
+            const float* rowp = vd.depth + (int64_t)(y < H ? y : H - 1) * W;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) px[i][c] = gload(rowp + (x + c < W ? x + c : W - 1));
+        }
     }
-    s_seg[row][seg] = m;
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+        const bool in = by * kTile1 + r0 + 32 * i < H;
+        float m = -kInf;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) m = fmaxf(m, in && x + c < W ? depth_key(px[i][c]) : -kInf);
+        m = fmaxf(m, __shfl_xor(m, 1));
+        m = fmaxf(m, __shfl_xor(m, 2));
+        if ((q & 3) == 0) s_seg[r0 + 32 * i][q >> 2] = m;
+    }
     __syncthreads();
     if (tid < 64) {
         const int ty = tid / (kTile1 / kTile0), tx = tid % (kTile1 / kTile0);
@@ -341,7 +362,14 @@ __device__ void depth_tiles(const VolDesc* __restrict__ vols, int nvol, uint32_t
     }
 }
 
-// The prep kernel: workgroups [0, pair_blocks) take the (node, brick) items;
+// The prep kernel.  Latency-bound up to about 250K items (a chain of
+// descriptor, node, list slot and bound): with the node's position, radius
+// and transform loaded together before the list atomic, the descriptor read
+// through the scalar cache and depth_tiles' loads all in flight it takes 9.6
+// us at 72x60x84 with 160 nodes (15.4 before) and 11.4 us at 250x262x246 with
+// 2048 nodes (16.9); at 512^3 with 4096 nodes (393K items of 8x8x4 bricks) the
+// two atomics an item bound it, 18.5 us.
+// Workgroups [0, pair_blocks) take the (node, brick) items;
 // workgroups [pair_blocks, gridDim.x) compute the depth-tile maxima of the
 // screened volumes' frames instead (one 128 x 128 pixel block each).
 template <class S>
@@ -360,15 +388,15 @@ __global__ __launch_bounds__(kPrepThreads) void k_prep_bin(
     for (int v = threadIdx.x; v < nvol; v += blockDim.x) s_k1[v] = vols[v].k1_base;
 
     // Clear the collision tiles the previous frame on this workspace flagged
-    // (tiles [0, clear_tiles) hold every flag it can have set).
-    for (uint32_t t = gid; t < clear_tiles; t += nthreads) {
-        if (tile_flag[t]) {
-            uint4* w = (uint4*)(bitmap + (uint64_t)t * 32u);
+    // (tiles [0, clear_tiles) hold every flag it can have set).  The first
+    // flag's load is waited for only after the node items.
+    const auto clear_tile = [&](uint32_t t) {
+        uint4* w = (uint4*)(bitmap + (uint64_t)t * 32u);
 #pragma unroll
-            for (int k = 0; k < 8; ++k) w[k] = make_uint4(0u, 0u, 0u, 0u);
-            tile_flag[t] = 0u;
-        }
-    }
+        for (int k = 0; k < 8; ++k) w[k] = make_uint4(0u, 0u, 0u, 0u);
+        tile_flag[t] = 0u;
+    };
+    const uint32_t flag0 = gid < clear_tiles ? tile_flag[gid] : 0u;
     if (gid < kStCount * kStatSlots) stat[gid] = 0ull;
     if (gid == 0) {
         ctrl->overflow_records = 0u;
@@ -380,9 +408,9 @@ __global__ __launch_bounds__(kPrepThreads) void k_prep_bin(
     // list, recorded as (brick, node << 7 | slot) for the list fill once
     // k_compact has placed every list in the pool ({kNone, 0}: no entry).
     uint2 entry = make_uint2(kNone, 0u);
-    do {
-        if (gid >= total) break;
-        int v = 0, hi = nvol - 1;  // last volume whose first item is <= gid
+    int v = 0;
+    if (gid < total) {
+        int hi = nvol - 1;  // last volume whose first item is <= gid
         while (v < hi) {
             const int mid = (v + hi + 1) >> 1;
             if (s_k1[mid] <= gid)
@@ -390,19 +418,32 @@ __global__ __launch_bounds__(kPrepThreads) void k_prep_bin(
             else
                 hi = mid - 1;
         }
-        const VolDesc& vd = vols[v];
+    }
+    const auto bin_item = [&](const VolDesc& vd) {
         const uint32_t local = gid - vd.k1_base;
-        if (local >= vd.k1_count) break;
+        if (local >= vd.k1_count) return;
         const uint32_t nb = (uint32_t)(vd.maxb[0] * vd.maxb[1] * vd.maxb[2]);
         const uint32_t j = local / nb;
         const uint32_t o = local - j * nb;
 
         // translateKernel(nodes, -c), src/VolumeFusion.cu:708
+        // the node's position, radius and transform in one round of loads
         const float* np = vd.nodes + 3ull * j;
+        const float n0 = gload(np), n1 = gload(np + 1), n2 = gload(np + 2);
+        const float r = gload(vd.radii + j);
+        float M[16];  // column-major: T(a, i) = M[4 i + a]
+        if (vd.T && (vd.screen || o == 0)) {
+            const float* Tp = vd.T + 16ull * j;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) M[i] = gload(Tp + i);
+        } else {  // the knn-only entry point has no transforms
+#pragma unroll
+            for (int i = 0; i < 16; ++i) M[i] = i % 5 == 0 ? 1.0f : 0.0f;
+        }
         float m[3];
-        m[0] = np[0] + (-vd.c[0]);
-        m[1] = np[1] + (-vd.c[1]);
-        m[2] = np[2] + (-vd.c[2]);
+        m[0] = n0 + (-vd.c[0]);
+        m[1] = n1 + (-vd.c[1]);
+        m[2] = n2 + (-vd.c[2]);
         // cube corner, src/TSDFWarp.cu:46-48
         int32_t nv[3];
         world_to_voxel(vd.g, m, nv);
@@ -415,7 +456,6 @@ __global__ __launch_bounds__(kPrepThreads) void k_prep_bin(
             lo[a] = (int32_t)l;
         }
         if (o == 0) {
-            const float r = vd.radii[j];
             const float rr = r * r;
             const float den = 2.0f * rr;
             NodeRec rec;
@@ -423,17 +463,12 @@ __global__ __launch_bounds__(kPrepThreads) void k_prep_bin(
             rec.lo = make_int4(lo[0], lo[1], lo[2], 0);
             if (vd.T && vd.blend == VF_BLEND_DQB) {
                 // t0, t1: the node's dual quaternion (real, dual)
-                mat4_to_dq(vd.T + 16ull * j, &rec.t0, &rec.t1);
+                mat4_to_dq(M, &rec.t0, &rec.t1);
                 rec.t2 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            } else if (vd.T) {  // the knn-only entry point has no transforms
-                const float* M = vd.T + 16ull * j;
+            } else {
                 rec.t0 = make_float4(M[0], M[4], M[8], M[12]);
                 rec.t1 = make_float4(M[1], M[5], M[9], M[13]);
                 rec.t2 = make_float4(M[2], M[6], M[10], M[14]);
-            } else {
-                rec.t0 = make_float4(1.0f, 0.0f, 0.0f, 0.0f);
-                rec.t1 = make_float4(0.0f, 1.0f, 0.0f, 0.0f);
-                rec.t2 = make_float4(0.0f, 0.0f, 1.0f, 0.0f);
             }
             rec.w = make_float4(den, 1.0f / den, 0.0f, 0.0f);
             nrec[vd.node_base + j] = rec;
@@ -451,12 +486,12 @@ __global__ __launch_bounds__(kPrepThreads) void k_prep_bin(
             blo[a] = (int32_t)(l / bs[a]);
             bhi[a] = (int32_t)(h / bs[a]);
         }
-        if (empty) break;
+        if (empty) return;
         const int32_t ox = (int32_t)(o % (uint32_t)vd.maxb[0]);
         const int32_t oy = (int32_t)((o / (uint32_t)vd.maxb[0]) % (uint32_t)vd.maxb[1]);
         const int32_t oz = (int32_t)(o / (uint32_t)(vd.maxb[0] * vd.maxb[1]));
         const int32_t bx = blo[0] + ox, by = blo[1] + oy, bz = blo[2] + oz;
-        if (bx > bhi[0] || by > bhi[1] || bz > bhi[2]) break;
+        if (bx > bhi[0] || by > bhi[1] || bz > bhi[2]) return;
         const uint32_t b = ((uint32_t)bz * (uint32_t)vd.bdim[1] + (uint32_t)by) * (uint32_t)vd.bdim[0] + (uint32_t)bx;
         const uint32_t gb = vd.brick_base + b;
         const uint32_t slot = atomicAdd(brick_count + gb, 1u);
@@ -474,10 +509,23 @@ __global__ __launch_bounds__(kPrepThreads) void k_prep_bin(
                 if (h > vd.g.dim[a] - 1) h = vd.g.dim[a] - 1;
                 vhi[a] = (int32_t)h;
             }
-            atomicMax(brick_disp + gb, disp_bound_bits(vd, vd.T + 16ull * j, m, vd.radii[j], vlo, vhi));
+            atomicMax(brick_disp + gb, disp_bound_bits(vd, M, m, r, vlo, vhi));
         }
-    } while (false);
+    };
+    // A volume's items are contiguous, so a wave's lanes share their volume
+    // but at the volumes' borders: one volume at a time, its descriptor read
+    // through the scalar cache.
+    unsigned long long todo = __ballot(gid < total);
+    while (todo) {
+        const int vu = __builtin_amdgcn_readlane(v, __ffsll((long long)todo) - 1);
+        const bool mine = gid < total && v == vu;
+        todo &= ~__ballot(mine);
+        if (mine) bin_item(vols[vu]);
+    }
     if (gid < total) items[gid] = entry;
+    if (flag0) clear_tile(gid);
+    for (uint64_t t = (uint64_t)gid + nthreads; t < clear_tiles; t += nthreads)
+        if (tile_flag[t]) clear_tile((uint32_t)t);
 }
 
 // The frame's active bricks (those with a non-empty node list), in brick
@@ -865,13 +913,14 @@ __global__ __launch_bounds__(kPrepThreads) void k_fill_lists(const uint2* __rest
 // cleared for the next frame.  A group of kGrp lanes takes one candidate
 // (lane q tests tiles q, q + 8, ...); a workgroup takes kSelPerBlock
 // candidates at a time, in list order, so the active list keeps the
-// candidates' order.  The workgroups also fill the node lists.
+// candidates' order.  Workgroups [sel_blocks, gridDim.x) fill the node lists
+// beside the selection instead.
 constexpr uint32_t kSelPerRound = kPrepThreads / kGrp;
 constexpr uint32_t kSelPerBlock = kCompactPer * kSelPerRound;
 
 __global__ __launch_bounds__(kPrepThreads) void k_select(
-    const VolDesc* __restrict__ vols, const uint32_t* __restrict__ cand, const uint4* __restrict__ cand_info,
-    uint32_t* __restrict__ brick_count, uint32_t* __restrict__ brick_disp, const uint32_t* __restrict__ tile_mark,
+    const VolDesc* __restrict__ vols, int nvol, uint32_t sel_blocks, const uint32_t* __restrict__ cand,
+    const uint4* __restrict__ cand_info, uint32_t* __restrict__ brick_count, uint32_t* __restrict__ brick_disp, const uint32_t* __restrict__ tile_mark,
     const uint32_t* __restrict__ vol_mark, uint32_t* __restrict__ active2, uint2* __restrict__ active_oc2,
     Ctrl* __restrict__ ctrl, uint64_t brick_cap, int parity_arg, const uint2* __restrict__ items, uint32_t total_items,
     const uint32_t* __restrict__ brick_off, uint32_t* __restrict__ brick_nodes, unsigned long long* __restrict__ stat,
@@ -879,16 +928,23 @@ __global__ __launch_bounds__(kPrepThreads) void k_select(
     __shared__ uint32_t s_cnt[kCompactPer * kCompactWaves];
     __shared__ uint32_t s_base;
     __shared__ unsigned long long s_drop;
+    __shared__ int4 s_vd[kMaxBatch];  // per volume: first brick, first tile, tiles per row and column
+    if (blockIdx.x >= sel_blocks) {
+        fill_lists(items, total_items, brick_off, brick_nodes, (blockIdx.x - sel_blocks) * blockDim.x + threadIdx.x,
+                   (gridDim.x - sel_blocks) * blockDim.x);
+        return;
+    }
     if (threadIdx.x == 0) s_drop = 0ull;
-    fill_lists(items, total_items, brick_off, brick_nodes, blockIdx.x * blockDim.x + threadIdx.x,
-               gridDim.x * blockDim.x);
+    for (int v = threadIdx.x; v < nvol; v += blockDim.x)
+        s_vd[v] = make_int4((int)vols[v].brick_base, (int)vols[v].tile_base, vols[v].tdim[0], vols[v].tdim[1]);
+    __syncthreads();
     const uint32_t parity = frame_parity(ctrl, parity_arg);
     const uint32_t n = run_length(ctrl->cand_run[parity]);
     const uint32_t tag = ctrl->frame + 1u;
     const int q = (int)(threadIdx.x % kGrp);
     uint32_t dropped = 0;
     // the loop bound is the same for every thread of the workgroup
-    for (uint64_t c0 = (uint64_t)blockIdx.x * kSelPerBlock; c0 < n; c0 += (uint64_t)gridDim.x * kSelPerBlock) {
+    for (uint64_t c0 = (uint64_t)blockIdx.x * kSelPerBlock; c0 < n; c0 += (uint64_t)sel_blocks * kSelPerBlock) {
         uint32_t flags = 0, items[kCompactPer];
         uint2 ocs[kCompactPer];
 #pragma unroll
@@ -900,8 +956,8 @@ __global__ __launch_bounds__(kPrepThreads) void k_select(
             const uint32_t item = cand[i];
             const uint4 info = cand_info[i];
             const uint32_t v = item >> 24;
-            const VolDesc& vd = vols[v];
-            const uint32_t gb = vd.brick_base + (item & 0xffffffu);
+            const int4 vd = s_vd[v];
+            const uint32_t gb = (uint32_t)vd.x + (item & 0xffffffu);
             bool keep;
             if (info.w & (kScPend | kScAll | kScKeep)) {
                 keep = true;
@@ -923,7 +979,7 @@ __global__ __launch_bounds__(kPrepThreads) void k_select(
                     m[u] = 0u;
                     if (t < nt) {
                         const uint32_t tz = z0 + t / nxy, ty = y0 + (t % nxy) / nx, tx = x0 + t % nx;
-                        m[u] = tile_mark[vd.tile_base + (tz * (uint32_t)vd.tdim[1] + ty) * (uint32_t)vd.tdim[0] + tx];
+                        m[u] = tile_mark[(uint32_t)vd.y + (tz * (uint32_t)vd.w + ty) * (uint32_t)vd.z + tx];
                     }
                 }
                 bool hit = false;
@@ -1929,6 +1985,7 @@ struct FrameSetup {
     bool screen = false;        // some volume is screened: k_compact feeds k_select
     uint64_t blocks_pair = 0;   // k_prep_bin workgroups over (node, brick) pairs
     uint64_t blocks_pyr = 0;    // k_prep_bin workgroups over depth blocks
+    uint64_t blocks_fill = 0;   // k_select workgroups that fill the node lists
     uint32_t k1 = 0;
     uint64_t blocks_prep = 0, blocks_a = 0, blocks_b = 0, blocks_redo = 0, arena_cap = 0, overflow_cap = 0, bricks = 0;
     bool redo = false;         // launch the redo pass (a record budget: some bricks may not fit)
@@ -2170,6 +2227,8 @@ int setup_frame(vf_workspace* ws, int nvol, const vf_volume* vols, const vf_grap
     fs->k1 = (uint32_t)k1;
     fs->blocks_pair = std::max<uint64_t>((k1 + kPrepThreads - 1) / kPrepThreads, 256);
     fs->blocks_pyr = pyr_blk;
+    // four items a thread in one round, at most two workgroups a CU
+    fs->blocks_fill = std::min<uint64_t>((k1 + 4 * kPrepThreads - 1) / (4 * kPrepThreads) + 1, (uint64_t)cus * 2);
     fs->blocks_prep = fs->blocks_pair + fs->blocks_pyr;
     fs->screen = any_screen;
     fs->blocks_a = blocks_a;
@@ -2205,7 +2264,12 @@ int launch_kernels_shape(Buffers& B, const FrameSetup& fs, int parity_arg, KnnOu
                (const float*)B.dmax, B.active, B.active_oc, B.cand, B.cand_info, B.tile_mark, B.vol_mark, B.ctrl,
                B.brick_cap, parity_arg);
         VF_LAUNCH_CHECK("k_compact");
-        launch(k_select, grid_c, dim3(kPrepThreads), stream, nullptr, e[1], vols, (const uint32_t*)B.cand,
+        // selection: as many workgroups as the compaction, at least eight
+        // where there are bricks for them (a small volume's candidates in one
+        // round)
+        const unsigned sel = std::max<unsigned>(grid_c.x, (unsigned)std::min<uint64_t>(8, (fs.bricks + 255) / 256));
+        launch(k_select, dim3(sel + (unsigned)fs.blocks_fill), dim3(kPrepThreads), stream, nullptr, e[1], vols,
+               fs.nvol, sel, (const uint32_t*)B.cand,
                (const uint4*)B.cand_info, B.brick_count, B.brick_disp, (const uint32_t*)B.tile_mark,
                (const uint32_t*)B.vol_mark, B.active, B.active_oc, B.ctrl, B.brick_cap, parity_arg,
                (const uint2*)B.items,
