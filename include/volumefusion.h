@@ -406,7 +406,9 @@ typedef struct vf_tuning {
     int32_t flags;            /* VF_TUNE_NO_SCREEN: sweep every brick with a node list */
 } vf_tuning;
 
-/* Tuning used by later vf_warped_integrate* calls on this workspace. */
+/* Tuning used by later vf_warped_integrate* calls on this workspace.  Until
+ * it is called the brick shape follows the batch's size (8x8x4 from 8M voxels
+ * on, 16x8x4 below; always 16x8x4 with a record budget). */
 int vf_workspace_set_tuning(vf_workspace* ws, const vf_tuning* tuning);
 
 /* Pending-record budget of later frames on this workspace (no counterpart in

@@ -444,3 +444,33 @@ def test_batch_mixes_blend_modes(vf, oracle):
                             s.cube, s.center, s.depth(0), s.delta, s.intrinsics(), s.max_weight, blend=b)
         np.testing.assert_array_equal(t.tsdf.download(), t_or)
         np.testing.assert_array_equal(t.weights.download(), w_or)
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (3, 2), (5, 129), (128, 128), (129, 16), (131, 127), (260, 140)])
+def test_screen_depth_tiles_at_frame_edges(vf, oracle, w, h):
+    """The brick screen's depth tiles on frames of one pixel up to a few
+    128-pixel blocks, widths on and off the 16-byte loads: bits equal the
+    oracle's, which knows no screen."""
+    f = 0.79 * max(w, h)
+    cam = scenes.Camera(w, h, f, f, w / 2, h / 2)
+    run_frames(vf, oracle, scenes.small_scene(seed=w, k=4, cam=cam), [0, 1])
+
+
+@pytest.mark.parametrize("dim,bricks", [((256, 256, 128), (8, 8, 4)), ((256, 255, 128), (16, 8, 4))])
+def test_default_brick_shape_by_size(vf, dim, bricks):
+    """A workspace nobody tuned takes 8x8x4 bricks from 2^23 voxels on and
+    16x8x4 below; either way the bits are those of explicit 16x8x4 bricks."""
+    s = scenes.small_scene(seed=3, dim=dim, nodes=300, k=4, vs=0.003, radius=0.02)
+    out = []
+    for tuning in (None, (0, 0), ([(16, 8, 4), (16, 4, 4), (8, 8, 4)].index(bricks), 0)):
+        tsdf = ops.DeviceTsdf(s.size, s.dim, center=s.center, delta=s.delta)
+        graph = ops.DeviceMotionGraph(s.nodes, s.transforms(0), s.radii)
+        ws = ops.Workspace()
+        if tuning is not None:
+            ws.set_tuning(*tuning)
+        ops.warped_integrate(ws, tsdf, graph, dev(s.depth(0)), s.intrinsics(), s.k, s.delta, s.max_weight, s.cube)
+        out.append((tsdf.tsdf.download(), tsdf.weights.download(), ws.last_stats()))
+    assert out[0][2]["updated"] > 0
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+    assert out[0][2] == out[2][2]

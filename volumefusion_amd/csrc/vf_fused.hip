@@ -1769,6 +1769,7 @@ struct vf_workspace {
     std::vector<hipEvent_t> events;
     int timed_frames = 0;
     vf_tuning tuning = {0, 0, 0.0f, 0};
+    bool tuned = false;  // vf_workspace_set_tuning chose the brick shape
     // pending-record budget in records per voxel (0: the worst case); with a
     // budget the buffers grow to exactly what a frame needs
     float record_ratio = 0.0f;
@@ -2348,6 +2349,33 @@ int launch_kernels(vf_workspace* ws, const FrameSetup& fs, int parity_arg, KnnOu
     }
 }
 
+// The brick shape of a batch nobody tuned: 8x8x4 from 8M voxels on, 16x8x4
+// below.  Measured over volumes of 0.2M to 134M voxels, 100 to 4096 nodes and
+// both blends: the smaller bricks fit the supported shell more closely and
+// keep five workgroups on a CU, which pays once the bricks outnumber the
+// chip's workgroup slots (16x8x4 against 8x8x4, us per frame: 250x262x246 119
+// and 112, 348x383x400 157 and 134, 512^3 253 and 214, 16 volumes of 64^3 to
+// 384^3 543 and 416; 204x197x211, 8.5M voxels, 90 and 91); below that a frame
+// is a chain of latencies and twice the bricks only add to it (92x88x84 62
+// and 67, 158x163x152 74 and 82).
+// A batch whose cubes meet 2^28 smaller bricks or more keeps 16x8x4, so that
+// it stays within the (node, brick) item limit it had.
+int default_shape(int nvol, const vf_volume* vols, const vf_graph* graphs, const vf_warp_params* p) {
+    double voxels = 0.0, items = 0.0;
+    for (int v = 0; v < nvol; ++v) {
+        const int32_t d[3] = {vols[v].dim.x, vols[v].dim.y, vols[v].dim.z};
+        const int32_t c[3] = {p[v].voxels_per_node.x, p[v].voxels_per_node.y, p[v].voxels_per_node.z};
+        double n = 1.0, b = (double)graphs[v].count;
+        for (int a = 0; a < 3; ++a) {
+            n *= (double)std::max(d[a], 0);
+            b *= std::max(c[a], 1) / kShapeDims[2][a] + 2.0;
+        }
+        voxels += n;
+        items += b;
+    }
+    return voxels >= 0x1p23 && items < 0x1p28 ? 2 : 0;
+}
+
 // At least `frames` timed frames' events exist (created in doubling steps).
 int grow_events(vf_workspace* ws, int frames) {
     const size_t want = (size_t)kTimedEvents * (size_t)frames;
@@ -2362,7 +2390,10 @@ int grow_events(vf_workspace* ws, int frames) {
 int launch_frame(vf_workspace* ws, int nvol, const vf_volume* vols, const vf_graph* graphs, const vf_frame* frames,
                  const vf_warp_params* p, bool knn_only, KnnOut kout, hipStream_t stream) {
     FrameSetup fs;
-    int st = setup_frame(ws, nvol, vols, graphs, frames, p, knn_only, ws->tuning, &fs, stream);
+    vf_tuning tuning = ws->tuning;
+    // (a record budget's owner sizes the workspace for 16x8x4 bricks)
+    if (!ws->tuned && ws->record_ratio == 0.0f) tuning.brick_shape = default_shape(nvol, vols, graphs, p);
+    int st = setup_frame(ws, nvol, vols, graphs, frames, p, knn_only, tuning, &fs, stream);
     if (st) return st;
     hipEvent_t* ev = nullptr;
     if (ws->timing && !knn_only) {
@@ -2717,6 +2748,7 @@ int vf_workspace_set_tuning(vf_workspace* ws, const vf_tuning* tuning) {
     int st = check_tuning(*tuning);
     if (st) return st;
     ws->tuning = *tuning;
+    ws->tuned = true;
     return VF_OK;
 }
 
@@ -2753,7 +2785,10 @@ int vf_plan_create(vf_plan** out, int n, const vf_volume* volumes, const vf_grap
     } else {
         std::lock_guard<std::mutex> lock(g_tune_mutex);
         auto it = g_tune_cache.find(tune_key(n, volumes, graphs, params));
-        if (it != g_tune_cache.end()) pl->tuning = it->second;
+        if (it != g_tune_cache.end())
+            pl->tuning = it->second;
+        else
+            pl->tuning.brick_shape = default_shape(n, volumes, graphs, params);
     }
     int st = plan_setup(pl, (hipStream_t)stream);
     if (st) {
