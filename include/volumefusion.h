@@ -533,9 +533,10 @@ int vf_gn_normal_equations(vf_workspace* ws, float* JTJ, float* JTr, const float
 
 /* A solver for one ICP iteration: builds the rows and JTJ and factorises
  * JTJ once (its value does not change during the Gauss-Newton iterations):
- * by Cholesky, JTJ being symmetric positive definite, or, where that finds a
- * non-positive pivot, by the LU with partial pivoting the reference uses
- * (VF_ERR_SINGULAR on a zero pivot).  The problem's buffers must stay alive
+ * by Cholesky, JTJ being symmetric positive definite (sparse, in binary64; a
+ * dense binary32 one where JTJ's fill is nearly full or its condition number
+ * is beyond binary32), or, where that finds a non-positive pivot, by the LU
+ * with partial pivoting the reference uses (VF_ERR_SINGULAR on a zero pivot).  The problem's buffers must stay alive
  * and unchanged while it exists. */
 typedef struct vf_gn_solver vf_gn_solver;
 typedef struct vf_gn_report {
@@ -561,7 +562,10 @@ int vf_gn_solver_destroy(vf_gn_solver* solver);
  * from pending) and their energy (sum of squares in binary64, fixed order;
  * the reference sums in float in thrust's order); stops when the energy drops
  * by less than min_step; else commits pending to transforms (after the first
- * iteration), solves JTJ x = JTr, updates pending and re-warps the mesh.
+ * iteration), solves JTJ x = JTr, updates pending and re-warps the mesh.  With
+ * the sparse factorisation the residuals of the second iteration on are
+ * those of canon warped by pending in binary64, which the rounded warped mesh
+ * stands for.
  * Blocks; reads back one double per iteration and one int at the end.
  * VF_ERR_HIP if a triangular solve's wait for a solved block gave up (a
  * bounded poll; the solve's waves end regardless). */

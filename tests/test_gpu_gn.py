@@ -259,3 +259,108 @@ def test_gn_solver_singular_normal_matrix(vf):
     if rc == 0:
         L.load().vf_gn_solver_destroy(solver)
     assert rc == 7  # VF_ERR_SINGULAR
+
+
+def _solve(vf, p, iters, factor=0):
+    """(transforms, pending, report) of the solver's loop on problem p."""
+    G = p.graph.shape[0]
+    d = _Dev(p)
+    T0 = np.tile(np.eye(4, dtype=F).reshape(16), (G, 1))
+    dT, dP, warped = dev(T0), DeviceArray((G, 16), F), DeviceArray(p.canon.shape, F)
+    L.call("vf_warp_mesh", p.knn.shape[1], warped.ptr, d.canon.ptr, dT.ptr, d.knn.ptr, d.kw.ptr, p.canon.shape[0], G,
+           None)
+    solver, rep = C.c_void_p(), L.GNReport()
+    L.call("vf_gn_solver_create_ex", C.byref(solver), C.byref(d.desc), factor, None)
+    try:
+        L.call("vf_gn_solver_iterate", solver, dT.ptr, dP.ptr, warped.ptr, d.canon.ptr, p.canon.shape[0], d.dmesh.ptr,
+               iters, -1e30, C.byref(rep), None)
+    finally:
+        L.load().vf_gn_solver_destroy(solver)
+    return dT.download(), dP.download(), rep
+
+
+@pytest.mark.parametrize("G", [1, 2, 10, 11, 41, 64, 130])
+def test_gn_sparse_factor_tiles(vf, oracle, G):
+    """The sparse factorisation where its 64-column tiles begin and end: one
+    node, 60 and 66 unknowns (a tile with padding, two tiles), the first graph
+    that is divided (41 nodes), several parts; against the binary64 loop, with
+    the bound of test_gn_solver_loop."""
+    p = scenes.gn_problem(8, G=G, M=60 * G, warp_angle_deg=2.0, warp_translation=0.004)
+    T0 = np.tile(np.eye(4, dtype=F).reshape(16), (G, 1))
+    T_or, pend_or, _, _ = _oracle_loop(oracle, p, T0, 3, -1e30)
+    T_f, pend_f, _, _ = _oracle_loop(oracle, p, T0, 3, -1e30, float_lu=True)
+    T, pend, rep = _solve(vf, p, 3)
+    assert rep.iterations == 3 and rep.cholesky == 1
+    np.testing.assert_allclose(T, T_or, rtol=0, atol=3.0 * float(np.abs(T_f - T_or).max()) + 1e-6)
+    np.testing.assert_allclose(pend, pend_or, rtol=0, atol=3.0 * float(np.abs(pend_f - pend_or).max()) + 1e-6)
+
+
+def test_gn_sparse_factor_many_columns_a_level(vf):
+    """Ninety graphs far apart as one: more than 64 tile columns are
+    eliminated together, and every graph's transforms equal those it gets
+    alone, to the rounding of the stored transforms (2^-22: the solve is
+    binary64)."""
+    import dataclasses
+    G, M, n = 24, 700, 90
+    one = [scenes.gn_problem(20 + i % 3, G=G, M=M) for i in range(n)]
+    shift = [np.array([0.7 * (i % 9), 0.7 * (i // 9), 0.0], F) for i in range(n)]
+    parts = [dataclasses.replace(p, graph=p.graph + s, canon=p.canon + s, dmesh=p.dmesh + s)
+             for p, s in zip(one, shift)]
+
+    def cat(name, step=0):
+        a = [getattr(p, name) for p in parts]
+        if step:
+            a = [np.where(x == np.uint32(0xFFFFFFFF), x, x + np.uint32(step * i)) if x.dtype == np.uint32
+                 else x + np.int32(step * i) for i, x in enumerate(a)]
+        return np.ascontiguousarray(np.concatenate(a))
+
+    whole = dataclasses.replace(parts[0], graph=cat("graph"), T=cat("T"), gknn=cat("gknn", G), canon=cat("canon"),
+                                knn=cat("knn", G), kw=cat("kw"), corr=cat("corr", M), dmesh=cat("dmesh"),
+                                dnormals=cat("dnormals"))
+    T, pend, rep = _solve(vf, whole, 3)
+    assert rep.cholesky == 1
+    for i in (0, 1, 44, 63, 64, 89):
+        Ti, pi, _ = _solve(vf, parts[i], 3)
+        scale = max(1.0, float(np.abs(pi).max()))
+        np.testing.assert_allclose(pend[G * i:G * (i + 1)], pi, rtol=0, atol=2.0 ** -22 * scale)
+
+
+def test_gn_crowded_nodes(vf, oracle):
+    """Nodes that share rows with 65 and more others: the assembly with two
+    waves a node."""
+    p = scenes.gn_problem(9, G=110, M=9000, K=8, radius=0.3)
+    rng = np.random.default_rng(4)
+    p.knn[:, :] = rng.integers(0, 110, p.knn.shape).astype(np.uint32)
+    for r in range(p.knn.shape[0]):  # distinct slots
+        p.knn[r] = rng.choice(110, p.knn.shape[1], replace=False)
+    p.kw[:, :] = F(1.0 / p.knn.shape[1])
+    T0 = np.tile(np.eye(4, dtype=F).reshape(16), (110, 1))
+    T_or, pend_or, _, _ = _oracle_loop(oracle, p, T0, 2, -1e30)
+    T_f, pend_f, _, _ = _oracle_loop(oracle, p, T0, 2, -1e30, float_lu=True)
+    T, pend, rep = _solve(vf, p, 2)
+    np.testing.assert_allclose(pend, pend_or, rtol=0, atol=3.0 * float(np.abs(pend_f - pend_or).max()) + 1e-6)
+
+
+@pytest.mark.parametrize("kind", ["nearly_singular", "dense_fill"])
+def test_gn_dense_path_where_it_stays(vf, kind):
+    """Problems that keep the dense factorisation: parallel normals and a
+    regularisation weight near zero leave directions that binary32 does not
+    determine; points bound to random nodes couple every part of the graph, so
+    that the fill is dense (2.7M tile updates of 64^3).  The dense path's
+    residuals are the binary32 ones, so its first energy has the bits of the
+    solver that is told to take the LU."""
+    import dataclasses
+    if kind == "nearly_singular":
+        p = scenes.gn_problem(6, G=200, M=6000)
+        p = dataclasses.replace(p, wR=1e-4, dnormals=np.tile(np.array([0, 0, 1], F), (p.dnormals.shape[0], 1)))
+    else:
+        G, M = 2700, 7000
+        p = scenes.gn_problem(6, G=G, M=M, K=6)
+        perm = np.random.default_rng(3).permuted(np.tile(np.arange(G, dtype=np.uint32), (16, 1)), axis=1)
+        p.knn[:, :] = perm.reshape(-1)[:6 * M].reshape(M, 6)
+        p.kw[:, :] = F(1.0 / 6.0)
+    _, _, auto = _solve(vf, p, 1)
+    _, _, lu = _solve(vf, p, 1, factor=1)
+    assert auto.iterations == 1 and auto.energy[0] == lu.energy[0]
+    _, _, plain = _solve(vf, scenes.gn_problem(6, G=200, M=6000), 1)
+    assert plain.cholesky == 1

@@ -1,0 +1,78 @@
+// vf_gn_sparse.hpp -- the solver's sparse Cholesky factorisation of the
+// Gauss-Newton normal matrix (vf_gn_sparse.hip), shared with vf_gn.hip.
+#pragma once
+
+#include <vector>
+
+#include "vf_host.hpp"
+
+namespace vf {
+
+// The rows of one linearisation as vf_gn.hip lays them out on the device.
+struct GnRowLists {
+    uint32_t G;
+    uint32_t rows;            // rows of J: C depth rows, then 3 R regularisation rows a node
+    uint32_t C;
+    int K, R;
+    float wD, wR;
+    const int32_t* corr;
+    const uint32_t* knn;
+    const float* kw;
+    const float* normals;
+    const uint32_t* gknn;
+    const uint32_t* off;      // G + 1: each node's first entry of rows_of
+    const uint32_t* rows_of;  // each node's rows, ascending
+    uint64_t entries;         // room in rows_of (an upper bound of off[G])
+    const uint32_t* node8;    // members of each row
+    const float* j48;         // their Jacobian entries
+    const float* graph;       // node positions
+    uint32_t* bad;            // set where a limit is exceeded
+    uint32_t max_nbr;         // most distinct nodes sharing rows with one node
+};
+
+// The factorisation: host-side schedule and device buffers.
+struct SparseChol {
+    uint32_t G = 0, T = 0, W = 0;  // nodes, 64-column tiles, 64-bit words of a tile bitmap
+    uint32_t max_nbr = 0;          // most neighbours of one node (itself included)
+    uint64_t off_tiles = 0, updates = 0;
+    // per level: first position in the level order, panels, updates
+    std::vector<uint32_t> level_first, level_panels, level_updates;
+    void* blob = nullptr;   // the uploaded schedule
+    const uint32_t *so = nullptr, *colptr = nullptr, *rowidx = nullptr, *rank = nullptr, *order = nullptr,
+                   *ppanel = nullptr, *pupdate = nullptr, *rowptr = nullptr, *level = nullptr, *pads = nullptr;
+    const unsigned long long* bits = nullptr;
+    const uint2 *fwd = nullptr, *bwd = nullptr;
+    uint32_t npads = 0;
+    // T diagonal tiles (their factors' inverses), the off-diagonal ones by
+    // column; then the same transposed
+    double* tiles = nullptr;
+    double* tiles_t = nullptr;
+    float* jn = nullptr;      // entries x 6: each node's Jacobian entries in its rows, times their multiplicity
+    double* vec = nullptr;    // the allocation of what follows
+    double *rhs = nullptr, *y = nullptr, *x = nullptr;  // 64 T each, in elimination order
+    uint4* tagged = nullptr;  // 64 T solved values, each half with its solve's epoch
+    double* res = nullptr;    // residuals
+    // ticket, failure flag, pivot failure, norm bound of the inverse and
+    // largest diagonal entry (float bits)
+    int* sync = nullptr;
+    uint32_t* nbr = nullptr;  // neighbour lists (CSR), their offsets and counts
+    uint32_t* nbr_off = nullptr;
+    uint32_t epoch = 0;
+};
+
+void sparse_free(SparseChol* s);
+// Orders the nodes and plans the factorisation; *use = 0 where the fill makes
+// the dense factorisation the faster one.  Reads the neighbour lists back
+// (blocks).  A problem that exceeds a limit leaves its code in *bad_out.
+int sparse_analyse(SparseChol* s, const GnRowLists& r, int* use, uint32_t* bad_out, hipStream_t stream);
+// Builds JTJ's lower triangle in the tiles and factorises it; *good = 0 where
+// a pivot was not positive or too small a part of its diagonal (blocks).
+int sparse_factor(SparseChol* s, const GnRowLists& r, int* good, hipStream_t stream);
+// Residuals of every row: the depth rows from `warped` (first iteration) or,
+// with warped NULL, from canon warped by T; their sum of squares in *energy.
+int sparse_residuals(SparseChol* s, const GnRowLists& r, const float* warped, const float* canon, const float* dmesh,
+                     const float* T, double* part, double* energy, hipStream_t stream);
+// JTr from the residuals, x = JTJ^-1 JTr, T <- T - U of every node.
+int sparse_step(SparseChol* s, const GnRowLists& r, float* T, hipStream_t stream);
+
+}  // namespace vf
