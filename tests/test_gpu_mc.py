@@ -153,3 +153,33 @@ def test_default_workspace_entry(vf, oracle):
     L.call("vf_device_synchronize")
     assert counts.download()[0] == vo.shape[0]
     np.testing.assert_array_equal(mesh.download()[:vo.shape[0]], vo)
+
+
+@pytest.mark.parametrize("full", [False, True], ids=["vertices", "faces"])
+def test_mesh_larger_than_the_first_buffers(vf, oracle, full):
+    """A volume whose every cube has output: more vertices than the buffers of
+    the first extraction hold, so a second one of the counted size runs; the
+    same mesh as into one buffer of the worst case, and the capacity still
+    bounds it."""
+    dims = (34, 33, 35)
+    n = dims[0] * dims[1] * dims[2]
+    rng = np.random.default_rng(5)
+    t, w = dev(rng.normal(size=n).astype(F)), dev(np.ones(n, F))
+    vs, size = (0.01,) * 3, tuple(0.01 * d for d in dims)
+    ws = ops.Workspace()
+    v, f = ops.marching_cubes(ws, t, w, dims, vs, size, full=full)
+    assert v.shape[0] > max(1 << 16, 16 * 34 * 35)
+    cap = v.shape[0]
+    mesh, counts = DeviceArray((cap, 3), F), DeviceArray((2,), np.uint32)
+    counts.fill(0)
+    faces = DeviceArray((cap // 3 + 1, 3), np.int32)
+    if full:
+        L.call("vf_marching_cubes_full", ws.handle, mesh.ptr, counts.ptr, cap, faces.ptr, counts.ptr + 4, cap // 3 + 1,
+               t.ptr, w.ptr, L.i3(dims), L.f3(vs), L.f3(size), 0.0, None)
+        np.testing.assert_array_equal(f, faces.download()[:f.shape[0]])
+    else:
+        L.call("vf_marching_cubes_mesh", ws.handle, mesh.ptr, counts.ptr, cap, t.ptr, w.ptr, L.i3(dims), L.f3(vs),
+               L.f3(size), 0.0, None)
+    np.testing.assert_array_equal(v, mesh.download())
+    with pytest.raises(L.VFError):
+        ops.marching_cubes(ws, t, w, dims, vs, size, full=full, capacity=cap - 1)

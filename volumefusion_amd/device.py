@@ -79,10 +79,13 @@ class DeviceArray:
             L.call("vf_memcpy_h2d", self._ptr, a.ctypes.data_as(C.c_void_p), self.nbytes, self.stream.ptr)
             self.stream.synchronize()
 
-    def download(self) -> np.ndarray:
-        out = np.empty(self.shape, self.dtype)
-        if self.nbytes:
-            L.call("vf_memcpy_d2h", out.ctypes.data_as(C.c_void_p), self._ptr, self.nbytes, self.stream.ptr)
+    def download(self, rows: int | None = None) -> np.ndarray:
+        """The array on the host, or its first `rows` rows."""
+        if rows is not None and not 0 <= rows <= self.shape[0]:
+            raise ValueError(f"{rows} rows of {self.shape[0]}")
+        out = np.empty(self.shape if rows is None else (rows, *self.shape[1:]), self.dtype)
+        if out.nbytes:
+            L.call("vf_memcpy_d2h", out.ctypes.data_as(C.c_void_p), self._ptr, out.nbytes, self.stream.ptr)
         return out
 
     def fill(self, value) -> None:

@@ -255,23 +255,31 @@ def marching_cubes(ws: "Workspace", tsdf: DeviceArray, weights: DeviceArray, dim
         capacity = 15 * max(X - 2, 0) * max(Y - 2, 0) * max(Z - 2, 0) if full else \
             12 * max(X - 2, 0) * max(Y - 2, 0) * max(Z - 2, 0)
         capacity = max(min(capacity, 1 << 26), 1)
-    mesh = DeviceArray((capacity, 3), np.float32, stream)
     counts = DeviceArray((2,), np.uint32, stream)
-    counts.upload(np.zeros(2, np.uint32))
-    if full:
-        faces = DeviceArray((capacity // 3 + 1, 3), np.int32, stream)
-        L.call("vf_marching_cubes_full", ws.handle, mesh.ptr, counts.ptr, int(capacity), faces.ptr, counts.ptr + 4,
-               int(faces.shape[0]), tsdf.ptr, weights.ptr, L.i3(dims), L.f3(voxel_size), L.f3(volume_size),
-               float(iso), _s(stream))
-    else:
-        L.call("vf_marching_cubes_mesh", ws.handle, mesh.ptr, counts.ptr, int(capacity), tsdf.ptr, weights.ptr,
-               L.i3(dims), L.f3(voxel_size), L.f3(volume_size), float(iso), _s(stream))
-    _done(stream)
-    nv, nf = (int(x) for x in counts.download())
-    if nv > capacity:
-        raise L.VFError(6, "marching_cubes", f"{nv} vertices exceed the capacity {capacity}")
-    verts = mesh.download()[:nv]
-    return verts, (faces.download()[:nf] if full else None)
+    # Buffers for about eight sheets through the volume, and a second
+    # extraction of the counted size where the surface has more (the call
+    # counts beyond its capacity): allocating the worst case and reading all of
+    # it back took 27 ms at 128x126x131, where the extraction takes 0.06.
+    room = min(capacity, max(1 << 16, 16 * max(X * Y, Y * Z, X * Z)))
+    while True:
+        mesh = DeviceArray((room, 3), np.float32, stream)
+        counts.fill(0)
+        if full:
+            faces = DeviceArray((room // 3 + 1, 3), np.int32, stream)
+            L.call("vf_marching_cubes_full", ws.handle, mesh.ptr, counts.ptr, int(room), faces.ptr, counts.ptr + 4,
+                   int(faces.shape[0]), tsdf.ptr, weights.ptr, L.i3(dims), L.f3(voxel_size), L.f3(volume_size),
+                   float(iso), _s(stream))
+        else:
+            L.call("vf_marching_cubes_mesh", ws.handle, mesh.ptr, counts.ptr, int(room), tsdf.ptr, weights.ptr,
+                   L.i3(dims), L.f3(voxel_size), L.f3(volume_size), float(iso), _s(stream))
+        _done(stream)
+        nv, nf = (int(x) for x in counts.download())
+        if nv > capacity:
+            raise L.VFError(6, "marching_cubes", f"{nv} vertices exceed the capacity {capacity}")
+        if nv <= room:
+            break
+        room = nv
+    return mesh.download(nv), (faces.download(nf) if full else None)
 
 
 # ---------------------------------------------------------------------------
