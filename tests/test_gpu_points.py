@@ -121,6 +121,43 @@ def test_warp_points_fused(vf, oracle, k, blend):
     np.testing.assert_array_equal(out, oracle.warp_points(k, pts, nodes, radii, T, blend=blend))
 
 
+@pytest.mark.parametrize("G,radius,spread,offset", [
+    (1, 0.05, 0.3, 0.0),      # one node: a grid of a few cells
+    (300, 0.02, 0.3, 0.0),    # sparse lists, most points beyond every radius
+    (1500, 0.06, 0.3, 0.0),   # lists of a few dozen nodes
+    (4096, 0.02, 0.02, 0.0),  # every list overflows: the ring search
+    (700, 0.03, 0.3, 40.0),   # coordinates far larger than a cell
+    (5000, 0.004, 0.3, 0.0),  # the cell limit: cells wider than the radius
+])
+def test_warp_points_near_lists(vf, oracle, G, radius, spread, offset):
+    rng = np.random.default_rng(G)
+    nodes, radii, T, pts = random_graph(rng, G, 4001, spread)
+    radii = (radius * rng.uniform(0.5, 1.0, G)).astype(F)
+    nodes, pts = (nodes + F(offset)).astype(F), (pts + F(offset)).astype(F)
+    if G > 200:
+        radii[5], radii[6] = 0.0, -1.0
+        nodes[11], nodes[12] = np.nan, np.inf
+    pts[:40:2] = nodes[rng.integers(0, G, 20)]
+    # at a radius from a node along an axis, and outside the nodes' box
+    pts[1:41:2] = nodes[:20 if G >= 20 else 1] + np.eye(3, dtype=F)[0] * radii.max()
+    pts[100:103] = [[np.nan, 0, 0], [np.inf, 0, 0], [-1e30, 1e30, 0]]
+    pts[103:106] = offset + np.eye(3) * (spread + radius)
+    out = ops.warp_points(ops.Workspace(), 6, dev(pts), ops.DeviceMotionGraph(nodes, T, radii)).download()
+    np.testing.assert_array_equal(out, oracle.warp_points(6, pts, nodes, radii, T))
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, 1e-20])
+def test_warp_points_radii_without_lists(vf, oracle, bad):
+    rng = np.random.default_rng(3)
+    nodes, radii, T, pts = random_graph(rng, 90, 900)
+    if bad == 1e-20:
+        radii[:] = bad
+    else:
+        radii[4] = bad
+    out = ops.warp_points(ops.Workspace(), 4, dev(pts), ops.DeviceMotionGraph(nodes, T, radii)).download()
+    np.testing.assert_array_equal(out, oracle.warp_points(4, pts, nodes, radii, T))
+
+
 def test_golden_inputs_fused(vf, oracle):
     g = json.loads((GOLDEN / "motiongraph_warp.json").read_text())
     T = np.ascontiguousarray(np.array(g["transforms_row_major"], F).transpose(0, 2, 1).reshape(-1, 16))

@@ -2654,6 +2654,8 @@ int workspace_scratch(vf_workspace* ws, uint64_t bytes, void** ptr, hipStream_t 
     return VF_OK;
 }
 
+uint64_t workspace_scratch_size(const vf_workspace* ws) { return ws ? ws->scratch_bytes : 0; }
+
 }  // namespace vf
 
 extern "C" {

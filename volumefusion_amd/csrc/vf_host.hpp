@@ -62,6 +62,7 @@ inline int check_k(int k) {
 
 // Device scratch owned by a workspace (defined with the workspace).
 int workspace_scratch(vf_workspace* ws, uint64_t bytes, void** ptr, hipStream_t stream);
+uint64_t workspace_scratch_size(const vf_workspace* ws);  // what it holds now; 0 for NULL
 
 // What one volume adds, in bytes, to each buffer group of a workspace with a
 // record budget of records_per_voxel when a batch holds it: node records,
