@@ -77,3 +77,34 @@ def test_fused_ingest_equals_sequence(vf, oracle, bilateral):
     np.testing.assert_array_equal(res["normals"].download(), n_or)
     assert res["count"] == cnt_or
     np.testing.assert_array_equal(res["centroid"], c_or)
+
+
+@pytest.mark.parametrize("W,H,r,sigma_i", [
+    (1, 1, 1, 75.0), (3, 200, 5, 75.0), (64, 8, 2, 75.0), (65, 9, 9, 75.0), (130, 35, 3, 75.0), (129, 17, 4, 75.0),
+    (200, 41, 6, 75.0), (63, 33, 7, 75.0), (257, 64, 8, 75.0),
+    (130, 35, 5, 0.01),  # colour weights that differ between taps
+    (130, 35, 5, 0.25), (130, 35, 5, 0.2500001), (130, 35, 5, -75.0),  # |thr norm| around 1, and of either sign
+])
+def test_fused_ingest_bilateral_windows(vf, oracle, W, H, r, sigma_i):
+    """Smooth windows, windows over a step and over removed pixels, at the
+    edges of the filter's tiles."""
+    rng = np.random.default_rng(W * H)
+    x, y = np.meshgrid(np.arange(W), np.arange(H))
+    d = (0.9 + 2e-4 * x + 1e-4 * rng.normal(size=(H, W))).astype(F)
+    d[(x + y) % 97 > 80] += F(0.2)
+    d[rng.random((H, W)) < 0.003] = 0.0
+    d[:, 2 * W // 3: 3 * W // 4] = 0.0
+    d[H // 2, W // 2], d[0, 0] = np.nan, np.inf
+    K = np.array([500, 0, 0, 0, 500, 0, W / 2, H / 2, 1], F)
+    dd = dev(d)
+    res = ops.ingest_depth(ops.Workspace(), dd, K, threshold=1.3, bilateral=(r, sigma_i, 3.0, 0.025))
+    b_or = oracle.bilateral(oracle.filter_depth(d, 1.3), r, sigma_i, 3.0, 0.025)
+    m_or = oracle.depth_to_mesh(b_or, K)
+    if W > 2 and H > 2:
+        n_or = oracle.depth_normals(m_or, H, W, 1.3, 2.1)
+        m_or, b_or = oracle.remove_depth_without_normals(n_or, m_or, b_or)
+    np.testing.assert_array_equal(dd.download(), b_or)
+    np.testing.assert_array_equal(res["vertices"].download(), m_or)
+    c_or, cnt_or = oracle.depth_centroid(m_or)
+    assert res["count"] == cnt_or
+    np.testing.assert_array_equal(res["centroid"], c_or)

@@ -66,6 +66,9 @@ __global__ __launch_bounds__(kTileX* kTileY) void k_bilateral(float* __restrict_
                                                               int H, int W, int r, float norm, float thr,
                                                               float pre_thr, float pre_fill, BilateralTables tab) {
     __shared__ float tile[(kTileX + 2 * kMaxRadius) * (kTileY + 2 * kMaxRadius)];
+    __shared__ float s_clr[31];  // read at a lane's own index
+    if (threadIdx.y * kTileX + threadIdx.x < 31)
+        s_clr[threadIdx.y * kTileX + threadIdx.x] = (float)tab.clr[threadIdx.y * kTileX + threadIdx.x];
     const int sw = kTileX + 2 * r, sh = kTileY + 2 * r;
     const int x0 = blockIdx.x * kTileX - r, y0 = blockIdx.y * kTileY - r;
     for (int e = threadIdx.y * kTileX + threadIdx.x; e < sw * sh; e += kTileX * kTileY) {
@@ -95,12 +98,147 @@ __global__ __launch_bounds__(kTileX* kTileY) void k_bilateral(float* __restrict_
             if (diff > thr) continue;
             int q = cvt_i32_rz(__builtin_fabsf(diff * norm));
             if (q > 30 || q < 0) q = 30;
-            const float w = tab.g2d[ig] * (float)tab.clr[q];
+            const float w = tab.g2d[ig] * s_clr[q];
             acc = acc + p * w;
             wsum = wsum + w;
         }
     }
     out[(uint64_t)y * W + x] = acc / wsum;
+}
+
+// The filtered frame's filter where the colour weight is the same for every tap
+// that counts (|thr norm| < 1, as with the reference's sigma of 75 for depths in
+// metres) and no kept depth is near FLT_MAX, which stands for a removed one in
+// the tile: it is then beyond thr of any depth, and its product with a weight of
+// 0 is 0, so a tap needs no branch.
+//
+// A wave whose windows all lie within thr of their own pixels (max - min <= thr:
+// rounding is monotone) skips the test of each tap, and the sum of the weights is
+// the table's.  Bound by VALU: 6 instructions a tap, or 2 and half of one for the
+// minimum and maximum.  Each thread filters two pixels of a column, so the taps
+// are read from LDS once for both.  The order of every pixel's sum is
+// k_bilateral's: columns of the window, each downwards.
+constexpr int kUniX = 64, kUniY = 8, kUniRows = 2;
+
+struct UniformTables {
+    float w[(2 * kMaxRadius + 1) * (2 * kMaxRadius + 1)];
+    float wsum;
+};
+
+template <int R>
+__global__ __launch_bounds__(kUniX* kUniY / kUniRows) void k_bilateral_uniform(float* __restrict__ out,
+                                                                                const float* __restrict__ in, int H,
+                                                                                int W, float thr, float pre_thr,
+                                                                                UniformTables tab) {
+    constexpr int kd = 2 * R + 1, sw = kUniX + 2 * R, sh = kUniY + 2 * R;
+    __shared__ float tile[sw * sh];
+    const int x0 = blockIdx.x * kUniX - R, y0 = blockIdx.y * kUniY - R;
+    const int tid = threadIdx.y * kUniX + threadIdx.x;
+    for (int e = tid; e < sw * sh; e += kUniX * kUniY / kUniRows) {
+        int gx = x0 + e % sw, gy = y0 + e / sw;
+        gx = gx < 0 ? 0 : (gx >= W ? W - 1 : gx);
+        gy = gy < 0 ? 0 : (gy >= H ? H - 1 : gy);
+        tile[e] = filtered(in[(uint64_t)gy * W + gx], pre_thr, FLT_MAX);
+    }
+    __syncthreads();
+    const int x = blockIdx.x * kUniX + threadIdx.x, y = blockIdx.y * kUniY + threadIdx.y * kUniRows;
+    const float* t0 = tile + threadIdx.y * kUniRows * sw + threadIdx.x;  // first tap of the upper pixel
+    const float c0 = t0[R * sw + R], c1 = t0[(R + 1) * sw + R];
+    const bool out0 = c0 == FLT_MAX, out1 = c1 == FLT_MAX;
+    if (__all(out0 && out1)) {
+        if (x < W && y < H) out[(uint64_t)y * W + x] = __builtin_inff();
+        if (x < W && y + 1 < H) out[(uint64_t)(y + 1) * W + x] = __builtin_inff();
+        return;
+    }
+    float lo = t0[0], hi = lo;
+#pragma unroll 1
+    for (int a = 0; a < kd; ++a) {
+#pragma unroll
+        for (int b = 0; b <= kd; ++b) {
+            const float p = t0[b * sw + a];
+            lo = fminf(lo, p);
+            hi = fmaxf(hi, p);
+        }
+    }
+    float acc0 = 0.0f, acc1 = 0.0f, ws0 = tab.wsum, ws1 = tab.wsum;
+    if (__all((out0 && out1) || hi - lo <= thr)) {
+#pragma unroll 1
+        for (int a = 0; a < kd; ++a) {
+            float q[kd + 1];
+#pragma unroll
+            for (int b = 0; b <= kd; ++b) q[b] = t0[b * sw + a];
+#pragma unroll
+            for (int b = 0; b < kd; ++b) {
+                const float w = tab.w[a * kd + b];
+                acc0 = acc0 + q[b] * w;
+                acc1 = acc1 + q[b + 1] * w;
+            }
+        }
+    } else {
+        ws0 = ws1 = 0.0f;
+#pragma unroll 1
+        for (int a = 0; a < kd; ++a) {
+            float q[kd + 1];
+#pragma unroll
+            for (int b = 0; b <= kd; ++b) q[b] = t0[b * sw + a];
+#pragma unroll
+            for (int b = 0; b < kd; ++b) {
+                const float w = tab.w[a * kd + b];
+                const float w0 = __builtin_fabsf(c0 - q[b]) > thr ? 0.0f : w;
+                const float w1 = __builtin_fabsf(c1 - q[b + 1]) > thr ? 0.0f : w;
+                acc0 = acc0 + q[b] * w0;
+                acc1 = acc1 + q[b + 1] * w1;
+                ws0 = ws0 + w0;
+                ws1 = ws1 + w1;
+            }
+        }
+    }
+    if (x < W && y < H) out[(uint64_t)y * W + x] = out0 ? __builtin_inff() : acc0 / ws0;
+    if (x < W && y + 1 < H) out[(uint64_t)(y + 1) * W + x] = out1 ? __builtin_inff() : acc1 / ws1;
+}
+
+// The bilateral filter of the filtered frame (1 <= r <= kMaxRadius): the kernel
+// above where it applies.
+int bilateral_filtered(float* out, const float* in, int H, int W, int r, double sigma_i, double sigma_s, float thr,
+                       float pre_thr, hipStream_t s) {
+    BilateralTables tab;
+    memset(&tab, 0, sizeof(tab));
+    bilateral_tables(r, sigma_s, &tab);
+    const float norm = (float)(30 / (3 * sigma_i));
+    const bool uniform = std::fabs(thr * norm) < 1.0f && thr >= 0.0f && thr < 1.0e30f && pre_thr < 1.0e30f &&
+                         H <= 65535 * kUniY;  // the grid's rows
+    if (!uniform) {
+        hipLaunchKernelGGL(k_bilateral<true>, dim3((W + kTileX - 1) / kTileX, (H + kTileY - 1) / kTileY),
+                           dim3(kTileX, kTileY), 0, s, out, in, H, W, r, norm, thr, pre_thr, __builtin_inff(), tab);
+        VF_LAUNCH_CHECK("k_bilateral");
+        return VF_OK;
+    }
+    UniformTables uni;
+    memset(&uni, 0, sizeof(uni));
+    const int n = (2 * r + 1) * (2 * r + 1);
+    for (int i = 0; i < n; ++i) {
+        uni.w[i] = tab.g2d[i] * (float)tab.clr[0];
+        uni.wsum = uni.wsum + uni.w[i];
+    }
+    const dim3 grid((W + kUniX - 1) / kUniX, (H + kUniY - 1) / kUniY), block(kUniX, kUniY / kUniRows);
+#define VF_UNI(RR)                                                                                              \
+    case RR:                                                                                                    \
+        hipLaunchKernelGGL(k_bilateral_uniform<RR>, grid, block, 0, s, out, in, H, W, thr, pre_thr, uni);       \
+        break
+    switch (r) {
+        VF_UNI(1);
+        VF_UNI(2);
+        VF_UNI(3);
+        VF_UNI(4);
+        VF_UNI(5);
+        VF_UNI(6);
+        VF_UNI(7);
+        VF_UNI(8);
+        VF_UNI(9);
+    }
+#undef VF_UNI
+    VF_LAUNCH_CHECK("k_bilateral_uniform");
+    return VF_OK;
 }
 
 struct Intr {
@@ -212,20 +350,23 @@ __device__ __forceinline__ void centroid_block(const float p[3], bool in, double
     s_sum[t][2] = in ? (double)p[2] : 0.0;
     if (t == 0) *s_cnt = 0;
     __syncthreads();
-    if (in && p[2] > 1.e-4f) atomicAdd(s_cnt, 1u);
-    for (int s = 128; s >= 1; s >>= 1) {
-        if (t < s) {
-            s_sum[t][0] = s_sum[t][0] + s_sum[t + s][0];
-            s_sum[t][1] = s_sum[t][1] + s_sum[t + s][1];
-            s_sum[t][2] = s_sum[t][2] + s_sum[t + s][2];
+    const uint32_t points = (uint32_t)__popcll(__ballot(in && p[2] > 1.e-4f));
+    if (__lane_id() == 0 && points) atomicAdd(s_cnt, points);
+    __syncthreads();
+    // s = 128 and 64 by the first wave from LDS, the rest within it
+    if (t < 64) {
+        double q[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            q[a] = (s_sum[t][a] + s_sum[t + 128][a]) + (s_sum[t + 64][a] + s_sum[t + 192][a]);
+            for (int s = 32; s >= 1; s >>= 1) q[a] = q[a] + __shfl_down(q[a], s);
         }
-        __syncthreads();
-    }
-    if (t == 0) {
-        block_sums[3 * blockIdx.x] = s_sum[0][0];
-        block_sums[3 * blockIdx.x + 1] = s_sum[0][1];
-        block_sums[3 * blockIdx.x + 2] = s_sum[0][2];
-        block_counts[blockIdx.x] = *s_cnt;
+        if (t == 0) {
+            block_sums[3 * blockIdx.x] = q[0];
+            block_sums[3 * blockIdx.x + 1] = q[1];
+            block_sums[3 * blockIdx.x + 2] = q[2];
+            block_counts[blockIdx.x] = *s_cnt;
+        }
     }
 }
 
@@ -259,29 +400,52 @@ __global__ __launch_bounds__(kFinalThreads) void k_centroid_final(const double* 
     const uint32_t c = (nb + kFinalThreads - 1) / kFinalThreads;
     double q0 = 0.0, q1 = 0.0, q2 = 0.0;
     uint64_t cnt = 0;
-    for (uint32_t b = t * c; b < (t + 1) * c && b < nb; ++b) {
-        q0 = q0 + block_sums[3 * b];
-        q1 = q1 + block_sums[3 * b + 1];
-        q2 = q2 + block_sums[3 * b + 2];
-        cnt += block_counts[b];
+    // four blocks' loads in flight at a time
+    const uint32_t be = min((t + 1) * c, nb);
+    for (uint32_t b = t * c; b < be; b += 4) {
+        double l[4][3];
+        uint32_t lc[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t i = min(b + j, be - 1);
+            l[j][0] = block_sums[3 * i];
+            l[j][1] = block_sums[3 * i + 1];
+            l[j][2] = block_sums[3 * i + 2];
+            lc[j] = block_counts[i];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const bool in = b + j < be;
+            q0 = in ? q0 + l[j][0] : q0;
+            q1 = in ? q1 + l[j][1] : q1;
+            q2 = in ? q2 + l[j][2] : q2;
+            cnt += in ? lc[j] : 0u;
+        }
     }
     s_part[0][t] = q0;
     s_part[1][t] = q1;
     s_part[2][t] = q2;
     __syncthreads();
     if (cnt) atomicAdd(&s_cnt, (unsigned long long)cnt);
-    for (uint32_t s = kFinalThreads / 2; s >= 1; s >>= 1) {
+    for (uint32_t s = kFinalThreads / 2; s >= 64; s >>= 1) {
         if (t < s) {
 #pragma unroll
             for (int a = 0; a < 3; ++a) s_part[a][t] = s_part[a][t] + s_part[a][t + s];
         }
         __syncthreads();
     }
+    if (t >= 64) return;
+    double q[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        q[a] = s_part[a][t];
+        for (int s = 32; s >= 1; s >>= 1) q[a] = q[a] + __shfl_down(q[a], s);
+    }
     if (t == 0) {
         const uint64_t total = s_cnt;
-        out[0] = (float)s_part[0][0] / (float)total;
-        out[1] = (float)s_part[1][0] / (float)total;
-        out[2] = (float)s_part[2][0] / (float)total;
+        out[0] = (float)q[0] / (float)total;
+        out[1] = (float)q[1] / (float)total;
+        out[2] = (float)q[2] / (float)total;
         out[3] = __uint_as_float((uint32_t)total);  // count, bit pattern (frames are < 2^32 pixels)
     }
 }
@@ -476,14 +640,9 @@ int vf_ingest_depth(vf_workspace* ws, float* depth, int width, int height, vf_ma
     float* out = (float*)(counts + nb + (nb & 1));
     // 1. filter (and the bilateral filter of the filtered frame)
     if (bilateral_radius > 0) {
-        BilateralTables tab;
-        memset(&tab, 0, sizeof(tab));
-        bilateral_tables(bilateral_radius, sigma_s, &tab);
-        const float norm = (float)(30 / (3 * sigma_i));
-        dim3 grid((width + kTileX - 1) / kTileX, (height + kTileY - 1) / kTileY);
-        hipLaunchKernelGGL(k_bilateral<true>, grid, dim3(kTileX, kTileY), 0, s, depth_f, (const float*)depth, height,
-                           width, bilateral_radius, norm, bilateral_threshold, threshold, __builtin_inff(), tab);
-        VF_LAUNCH_CHECK("k_bilateral");
+        st = bilateral_filtered(depth_f, depth, height, width, bilateral_radius, sigma_i, sigma_s,
+                                bilateral_threshold, threshold, s);
+        if (st) return st;
     } else {
         VF_HIP(hipMemcpyAsync(depth_f, depth, n * 4, hipMemcpyDeviceToDevice, s));
         hipLaunchKernelGGL(k_filter_depth, dim3(g1(n)), dim3(256), 0, s, depth_f, n, threshold, __builtin_inff());
