@@ -400,27 +400,11 @@ __global__ __launch_bounds__(kFinalThreads) void k_centroid_final(const double* 
     const uint32_t c = (nb + kFinalThreads - 1) / kFinalThreads;
     double q0 = 0.0, q1 = 0.0, q2 = 0.0;
     uint64_t cnt = 0;
-    // four blocks' loads in flight at a time
-    const uint32_t be = min((t + 1) * c, nb);
-    for (uint32_t b = t * c; b < be; b += 4) {
-        double l[4][3];
-        uint32_t lc[4];
-#pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const uint32_t i = min(b + j, be - 1);
-            l[j][0] = block_sums[3 * i];
-            l[j][1] = block_sums[3 * i + 1];
-            l[j][2] = block_sums[3 * i + 2];
-            lc[j] = block_counts[i];
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const bool in = b + j < be;
-            q0 = in ? q0 + l[j][0] : q0;
-            q1 = in ? q1 + l[j][1] : q1;
-            q2 = in ? q2 + l[j][2] : q2;
-            cnt += in ? lc[j] : 0u;
-        }
+    for (uint32_t b = t * c; b < (t + 1) * c && b < nb; ++b) {
+        q0 = q0 + block_sums[3 * b];
+        q1 = q1 + block_sums[3 * b + 1];
+        q2 = q2 + block_sums[3 * b + 2];
+        cnt += block_counts[b];
     }
     s_part[0][t] = q0;
     s_part[1][t] = q1;
