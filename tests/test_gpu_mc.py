@@ -140,6 +140,25 @@ def test_append_after_count_and_capacity(vf, oracle):
     np.testing.assert_array_equal(fc[2:2 + k], fo[:k] + 5)
 
 
+@pytest.mark.parametrize("full", [False, True])
+@pytest.mark.parametrize("X,field", [(62, "checker"), (62, "noise"), (63, "noise"), (123, "noise"), (5, "noise")])
+def test_crowded_runs(vf, oracle, X, field, full):
+    """Runs of 60 cubes whose every cube has output: up to 720 vertices a run,
+    and runs of one, two or three cubes."""
+    dims = (X, 7, 19)
+    rng = np.random.default_rng(X)
+    z, y, x = np.meshgrid(*(np.arange(n) for n in dims[::-1]), indexing="ij")
+    sign = np.where((x + y + z) % 2, 1.0, -1.0) if field == "checker" else rng.choice([-1.0, 1.0], x.shape)
+    tsdf = (sign * rng.uniform(0.1, 1.0, x.shape)).astype(F).ravel()
+    wt = np.ones_like(tsdf)
+    vs, size = (F(0.01),) * 3, tuple(F(0.01) * F(n) for n in dims)
+    v, f = ops.marching_cubes(ops.Workspace(), dev(tsdf), dev(wt), dims, vs, size, full=full)
+    vo, fo = oracle.marching_cubes(tsdf, wt, dims, vs, size, full=full)
+    np.testing.assert_array_equal(v, vo)
+    if full:
+        np.testing.assert_array_equal(f, fo)
+
+
 def test_default_workspace_entry(vf, oracle):
     """A NULL workspace (the af:: shims' path) uses the device default."""
     tsdf, wt, dims, vs, size = sphere(16, 0.8 / 16, 0.27)
