@@ -4,6 +4,7 @@ inputs for that stage, so a mismatch names the stage."""
 import numpy as np
 import pytest
 
+from volumefusion_amd import _lib as L
 from volumefusion_amd import ops, scenes
 from volumefusion_amd.device import DeviceArray
 
@@ -310,3 +311,40 @@ def test_integrate_plain_and_camera_frame(vf, oracle):
                                                     tsdf.voxel_size(), s.size, Rw_cm, tw, I3, c, s.intrinsics(), 15.0)
     np.testing.assert_array_equal(tsdf.tsdf.download(), t2)
     np.testing.assert_array_equal(tsdf.weights.download(), w2)
+
+
+@pytest.mark.parametrize("camera", [False, True])
+@pytest.mark.parametrize("dim,shift", [
+    ((4, 1, 1), 0), ((4, 70, 3), 0), ((64, 33, 9), 0), ((100, 21, 40), 0), ((260, 17, 24), 0),  # four voxels a thread
+    ((64, 33, 9), 1), ((64, 33, 9), 2), ((62, 33, 9), 0), ((3, 3, 3), 0),                       # a voxel a thread
+])
+def test_integrate_plain_rows(vf, oracle, dim, shift, camera):
+    """Rows of whole quads and others, and volumes that start off 16 bytes."""
+    s = scenes.sphere128()
+    depth = s.depth(0)
+    depth[200:260:3, 250:400] = np.nan
+    H, W = depth.shape
+    n = dim[0] * dim[1] * dim[2]
+    vs = tuple(F(0.7) / F(d) for d in dim)
+    size = (F(0.7),) * 3
+    rng = np.random.default_rng(n)
+    t0, w0 = rng.uniform(-1, 1, n).astype(F), rng.integers(0, 17, n).astype(F)
+    c, th = np.array(s.center, F) + F(0.013), 0.2
+    R = np.array([np.cos(th), np.sin(th), 0, -np.sin(th), np.cos(th), 0, 0, 0, 1], F)
+    tw = np.array([0.01, -0.02, 0.03], F)
+    bt, bw = np.full(n + 8, 5, F), np.full(n + 8, 6, F)
+    bt[shift:shift + n], bw[shift:shift + n] = t0, w0
+    gt, gw, gd = dev(bt), dev(bw), dev(depth)
+    args = (L.f3(size), L.m3(R), L.f3(c), L.m3(s.intrinsics()), 15.0, None)
+    head = (gt.ptr + 4 * shift, gw.ptr + 4 * shift, gd.ptr, L.Int2(W, H), float(s.delta), L.i3(dim), L.f3(vs))
+    if camera:
+        t, w, _ = oracle.integrate_camera_frame(t0, w0, depth, s.delta, dim, vs, size, R, tw, R, c, s.intrinsics(),
+                                                15.0)
+        L.call("vf_integrate_tsdf_camera_frame", *head, args[0], L.m3(R), L.f3(tw), *args[1:])
+    else:
+        t, w, _ = oracle.integrate_plain(t0, w0, depth, s.delta, dim, vs, size, R, c, s.intrinsics(), 15.0)
+        L.call("vf_integrate_tsdf", *head, *args)
+    L.call("vf_device_synchronize")
+    bt[shift:shift + n], bw[shift:shift + n] = t, w
+    np.testing.assert_array_equal(gt.download(), bt)
+    np.testing.assert_array_equal(gw.download(), bw)

@@ -495,11 +495,9 @@ struct Camera {
     double rdelta;  // RN64(1 / delta)
 };
 
-// project3dToFrame + the tests of updateTsdf up to the read-modify-write,
-// src/TSDFIntegration.cu:16-58.  Returns the pixel index, or -1 when the
-// voxel is not updated; *tn is the new truncated sdf sample.
-__device__ __forceinline__ int64_t project_sample(const Camera& cam, const float* __restrict__ depth, const float p[3],
-                                                  float* tn) {
+// project3dToFrame, src/TSDFIntegration.cu:16-58: the pixel's index, or -1
+// behind the camera or outside the frame.
+__device__ __forceinline__ int64_t project_pixel(const Camera& cam, const float p[3]) {
     if (p[2] < 1.e-4f) return -1;
     const float zInv = rcp_rn(p[2]);
     const float ux = cam.fx * p[0];
@@ -509,13 +507,26 @@ __device__ __forceinline__ int64_t project_sample(const Camera& cam, const float
     const int32_t px = cvt_i32_rz(uf + 0.5f);
     const int32_t py = cvt_i32_rz(vf + 0.5f);
     if (px < 0 || px >= cam.W || py < 0 || py >= cam.H) return -1;
-    const int64_t pi = (int64_t)py * cam.W + px;
-    const float d = gload(depth + pi);
-    if (__builtin_isinf(d) || d < 1.e-4f) return -1;
-    const float sdf = p[2] - d;
-    if (sdf > cam.delta) return -1;
+    return (int64_t)py * cam.W + px;
+}
+
+// The tests of updateTsdf on the pixel's depth: false when the voxel is not
+// updated; *tn is the new truncated sdf sample.
+__device__ __forceinline__ bool depth_sample(const Camera& cam, float d, float z, float* tn) {
+    if (__builtin_isinf(d) || d < 1.e-4f) return false;
+    const float sdf = z - d;
+    if (sdf > cam.delta) return false;
     *tn = (sdf < -cam.delta) ? -1.0f : div_by_recip64(sdf, cam.delta, cam.rdelta);
-    return pi;
+    return true;
+}
+
+// Both, up to the read-modify-write.  Returns the pixel index, or -1 when the
+// voxel is not updated.
+__device__ __forceinline__ int64_t project_sample(const Camera& cam, const float* __restrict__ depth, const float p[3],
+                                                  float* tn) {
+    const int64_t pi = project_pixel(cam, p);
+    if (pi < 0) return -1;
+    return depth_sample(cam, gload(depth + pi), p[2], tn) ? pi : -1;
 }
 
 // The read-modify-write of updateTsdf, src/TSDFIntegration.cu:60-64: the
