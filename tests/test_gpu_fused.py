@@ -474,3 +474,15 @@ def test_default_brick_shape_by_size(vf, dim, bricks):
     np.testing.assert_array_equal(out[0][0], out[1][0])
     np.testing.assert_array_equal(out[0][1], out[1][1])
     assert out[0][2] == out[2][2]
+
+
+@pytest.mark.parametrize("shape", [0, 2, 3, 4])
+@pytest.mark.parametrize("nodes", [1, 63, 64, 65, 127, 128, 129])
+def test_brick_lists_around_a_wave(vf, oracle, nodes, shape):
+    """Brick lists of up to 128 entries in bricks of four and of eight waves
+    (129 spill): 64 entries are tested at a time."""
+    s = scenes.small_scene(seed=21, nodes=nodes, k=4)
+    rng = np.random.default_rng(nodes)
+    s.nodes[:] = s.nodes[:1] + rng.uniform(-0.006, 0.006, s.nodes.shape).astype(F)
+    st, gs = run_frames(vf, oracle, s, [0, 1], tuning=(shape, 0))
+    assert st["updated"] > 0 and (gs["overflow_bricks"] > 0) == (nodes > 128)
