@@ -362,55 +362,78 @@ __device__ int row_members(const GnRows& g, uint32_t row, Member* m) {
     return 2;
 }
 
-// Counts each node's rows; flags a member node outside the graph.
-__global__ void k_rows_count(GnRows g, uint32_t* __restrict__ cnt, uint32_t* __restrict__ bad) {
+// The nodes of mesh point ci's knn slots with a non-zero weight; kGnNone for
+// the others.  True where one of them lies outside the graph.
+__device__ __forceinline__ bool row_nodes(const GnRows& g, uint32_t ci, uint32_t id[kGnMaxK]) {
+    bool bad = false;
+    float w[kGnMaxK];
+#pragma unroll
+    for (int s = 0; s < kGnMaxK; ++s) {
+        w[s] = s < g.K ? g.kw[(uint64_t)g.K * ci + s] : 0.0f;
+        id[s] = s < g.K ? g.knn[(uint64_t)g.K * ci + s] : kGnNone;
+    }
+#pragma unroll
+    for (int s = 0; s < kGnMaxK; ++s) {
+        bad = bad || (w[s] != 0.0f && id[s] >= g.G);
+        if (w[s] == 0.0f) id[s] = kGnNone;
+    }
+    return bad;
+}
+
+// Counts each node's rows; flags a member node outside the graph.  A row's place
+// in a node's list is its atomic's result, which the fill reads (one atomic per
+// member; with a second counter in the fill the two took 134 and 142 us for 300K
+// points and 4096 nodes, and take 165 and 15).
+__global__ __launch_bounds__(256) void k_rows_count(GnRows g, uint32_t* __restrict__ cnt, uint32_t* __restrict__ place,
+                             uint32_t* __restrict__ bad) {
     const uint32_t rows = g.C + 3u * g.G * (uint32_t)g.R;
     const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
     if (row >= rows) return;
+    uint32_t* at = place + 8ull * row;
     if (row < g.C) {
         const uint32_t ci = (uint32_t)g.corr[2 * row];
-        for (int s = 0; s < g.K; ++s) {
-            if (g.kw[(uint64_t)g.K * ci + s] == 0.0f) continue;
-            const uint32_t j = g.knn[(uint64_t)g.K * ci + s];
-            if (j >= g.G) {
-                *bad = 1u;
-                continue;
-            }
-            atomicAdd(cnt + j, 1u);
-        }
+        uint32_t id[kGnMaxK], n[kGnMaxK];
+        if (row_nodes(g, ci, id)) *bad = 1u;
+#pragma unroll
+        for (int s = 0; s < kGnMaxK; ++s)
+            if (id[s] < g.G) n[s] = atomicAdd(cnt + id[s], 1u);
+#pragma unroll
+        for (int s = 0; s < kGnMaxK; ++s)
+            if (id[s] < g.G) at[s] = n[s];
         return;
     }
     const uint32_t mr = (row - g.C) / 3u;
     const uint32_t node = mr / (uint32_t)g.R, nb = g.gknn[mr];
     if (nb >= g.G) return;
-    atomicAdd(cnt + node, 1u);
-    if (nb != node) atomicAdd(cnt + nb, 1u);
+    at[0] = atomicAdd(cnt + node, 1u);
+    if (nb != node) at[1] = atomicAdd(cnt + nb, 1u);
 }
 
-__global__ void k_rows_fill(GnRows g, const uint32_t* __restrict__ off, uint32_t* __restrict__ fill,
+__global__ __launch_bounds__(256) void k_rows_fill(GnRows g, const uint32_t* __restrict__ off, const uint32_t* __restrict__ place,
                             uint32_t* __restrict__ rows_of) {
     const uint32_t rows = g.C + 3u * g.G * (uint32_t)g.R;
     const uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
     if (row >= rows) return;
+    const uint32_t* at = place + 8ull * row;
     if (row < g.C) {
         const uint32_t ci = (uint32_t)g.corr[2 * row];
-        for (int s = 0; s < g.K; ++s) {
-            if (g.kw[(uint64_t)g.K * ci + s] == 0.0f) continue;
-            const uint32_t j = g.knn[(uint64_t)g.K * ci + s];
-            if (j >= g.G) continue;
-            rows_of[off[j] + atomicAdd(fill + j, 1u)] = row;
-        }
+        uint32_t id[kGnMaxK];
+        row_nodes(g, ci, id);
+#pragma unroll
+        for (int s = 0; s < kGnMaxK; ++s)
+            if (id[s] < g.G) rows_of[off[id[s]] + at[s]] = row;
         return;
     }
     const uint32_t mr = (row - g.C) / 3u;
     const uint32_t node = mr / (uint32_t)g.R, nb = g.gknn[mr];
     if (nb >= g.G) return;
-    rows_of[off[node] + atomicAdd(fill + node, 1u)] = row;
-    if (nb != node) rows_of[off[nb] + atomicAdd(fill + nb, 1u)] = row;
+    rows_of[off[node] + at[0]] = row;
+    if (nb != node) rows_of[off[nb] + at[1]] = row;
 }
 
-// Sorts each node's row list (bitonic sort in LDS, one workgroup per node).
-__global__ __launch_bounds__(1024) void k_rows_sort(const uint32_t* __restrict__ off, uint32_t* __restrict__ rows_of,
+// Sorts each node's row list (bitonic sort in LDS, one workgroup per node; some
+// 540 rows a node: 83 us for 4096 nodes with four waves, 102 with sixteen).
+__global__ __launch_bounds__(256) void k_rows_sort(const uint32_t* __restrict__ off, uint32_t* __restrict__ rows_of,
                                                     uint32_t* __restrict__ bad) {
     __shared__ uint32_t s[kGnMaxRows];
     const uint32_t node = blockIdx.x;
@@ -977,7 +1000,6 @@ struct vf_gn_solver {
     uint64_t n = 0;  // 6 G
     // device buffers
     uint32_t* cnt = nullptr;   // G + 1: counts, then offsets
-    uint32_t* fill = nullptr;  // G
     uint32_t* rows_of = nullptr;
     uint32_t* node8 = nullptr;  // row data: members of each row
     float* j48 = nullptr;       // row data: their Jacobian entries
@@ -1009,7 +1031,7 @@ namespace vf {
 namespace {
 
 void gn_free(vf_gn_solver* s) {
-    void* ptrs[] = {s->cnt, s->fill, s->rows_of, s->node8, s->j48,  s->bad,  s->JTJ,   s->ipiv,
+    void* ptrs[] = {s->cnt, s->rows_of, s->node8, s->j48,  s->bad,  s->JTJ,   s->ipiv,
                     s->info, s->r,   s->x,       s->y,     s->perm, s->part, s->energy, s->chain, s->tagged};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -1072,9 +1094,14 @@ GnRows make_rows(const vf_gn_problem* p) {
 int build_rows(vf_gn_solver* s, hipStream_t st) {
     const GnRows& g = s->rows;
     VF_HIP(hipMemsetAsync(s->cnt, 0, sizeof(uint32_t) * (g.G + 1ull), st));
-    VF_HIP(hipMemsetAsync(s->fill, 0, sizeof(uint32_t) * g.G, st));
     VF_HIP(hipMemsetAsync(s->bad, 0, sizeof(uint32_t), st));
-    hipLaunchKernelGGL(k_rows_count, dim3(blocks_for(s->nrows, 256)), dim3(256), 0, st, g, s->cnt, s->bad);
+    if (!s->node8) {
+        int e = gn_alloc(&s->node8, 8ull * s->nrows);
+        if (!e) e = gn_alloc(&s->j48, 48ull * s->nrows);
+        if (e) return e;
+    }
+    uint32_t* place = (uint32_t*)s->j48;  // written before the rows' Jacobians
+    hipLaunchKernelGGL(k_rows_count, dim3(blocks_for(s->nrows, 256)), dim3(256), 0, st, g, s->cnt, place, s->bad);
     VF_LAUNCH_CHECK("k_rows_count");
     hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, s->cnt, g.G + 1u, (uint32_t*)nullptr);
     VF_LAUNCH_CHECK("k_scan_counts");
@@ -1085,15 +1112,10 @@ int build_rows(vf_gn_solver* s, hipStream_t st) {
     if (!s->rows_of) e = gn_alloc(&s->rows_of, s->entries);
     if (e) return e;
     hipLaunchKernelGGL(k_rows_fill, dim3(blocks_for(s->nrows, 256)), dim3(256), 0, st, g, (const uint32_t*)s->cnt,
-                       s->fill, s->rows_of);
+                       (const uint32_t*)place, s->rows_of);
     VF_LAUNCH_CHECK("k_rows_fill");
-    hipLaunchKernelGGL(k_rows_sort, dim3(g.G), dim3(1024), 0, st, (const uint32_t*)s->cnt, s->rows_of, s->bad);
+    hipLaunchKernelGGL(k_rows_sort, dim3(g.G), dim3(256), 0, st, (const uint32_t*)s->cnt, s->rows_of, s->bad);
     VF_LAUNCH_CHECK("k_rows_sort");
-    if (!s->node8) {
-        e = gn_alloc(&s->node8, 8ull * s->nrows);
-        if (!e) e = gn_alloc(&s->j48, 48ull * s->nrows);
-        if (e) return e;
-    }
     hipLaunchKernelGGL(k_row_data, dim3(blocks_for(s->nrows, 256)), dim3(256), 0, st, g, s->nrows, s->node8, s->j48,
                        s->bad);
     VF_LAUNCH_CHECK("k_row_data");
@@ -1444,7 +1466,6 @@ int vf_gn_normal_equations(vf_workspace* ws, float* JTJ, float* JTr, const float
     s.n = 6ull * s.rows.G;
     hipStream_t hs = (hipStream_t)stream;
     if (!st) st = gn_alloc(&s.cnt, s.rows.G + 1ull);
-    if (!st) st = gn_alloc(&s.fill, s.rows.G);
     if (!st) st = gn_alloc(&s.bad, 1);
     if (!st) st = build_rows(&s, hs);
     if (!st && JTJ) {
@@ -1480,7 +1501,6 @@ int vf_gn_solver_create_ex(vf_gn_solver** out, const vf_gn_problem* problem, int
     s->nrows = s->rows.C + 3u * s->rows.G * (uint32_t)s->rows.R;
     s->n = 6ull * s->rows.G;
     if (!st) st = gn_alloc(&s->cnt, s->rows.G + 1ull);
-    if (!st) st = gn_alloc(&s->fill, s->rows.G);
     if (!st) st = gn_alloc(&s->bad, 1);
     if (!st) st = gn_alloc(&s->r, s->nrows);
     if (!st) st = gn_alloc(&s->part, kEnergyBlocks);
