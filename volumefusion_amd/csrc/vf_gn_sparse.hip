@@ -205,7 +205,7 @@ __global__ __launch_bounds__(256) void k_sp_diagonal(const double* __restrict__ 
     if (__lane_id() == 0 && v > 0.0f) atomicMax(sync + 4, __float_as_int(v));
 }
 
-constexpr int kAsmRows = 4;  // rows in flight per wave
+constexpr int kAsmRows = 8;  // rows in flight per wave
 
 // The 6x6 blocks JTJ(i, j) of one node i and its neighbours j at or before it
 // in the elimination order, into the tiles, and the node's own Jacobian
@@ -215,7 +215,10 @@ constexpr int kAsmRows = 4;  // rows in flight per wave
 // products with the six entries of the row's own member (the last slot naming
 // i) to the member's block in the wave's LDS sums.  The waves' sums are added in
 // order.  Products are exact and sums binary64; the order differs from the
-// ascending one of the normal-equation entry point.
+// ascending one of the normal-equation entry point.  Bound by the latency of the
+// scattered row data, two workgroups a CU: with the next rows in flight 4096 nodes
+// of 300K points take 312 us, without 755 (reading, adding and writing the sums in
+// place of the LDS atomics was slower: 347 against 320, four rows in flight).
 __global__ __launch_bounds__(256) void k_sp_blocks(GnRowLists r, const uint32_t* __restrict__ nbr_off,
                                                    const uint32_t* __restrict__ nbr, Sched sc,
                                                    const uint32_t* __restrict__ so, uint32_t cap,
@@ -245,19 +248,33 @@ __global__ __launch_bounds__(256) void k_sp_blocks(GnRowLists r, const uint32_t*
     __syncthreads();
     const uint32_t b = r.off[i], n = r.off[i + 1] - b;
     const uint32_t q = (uint32_t)lane / 6u, c = (uint32_t)lane % 6u;
-    for (uint32_t e0 = kAsmRows * (uint32_t)wave; e0 < n; e0 += kAsmRows * waves) {
+    // the wave's share of the node's rows: 64 row numbers at a time, a lane each,
+    // and the next rows' data in flight while these are added
+    const uint32_t first = (uint32_t)((uint64_t)n * (uint32_t)wave / waves);
+    const uint32_t last = (uint32_t)((uint64_t)n * ((uint32_t)wave + 1u) / waves);
+    uint32_t ids = 0, vn[kAsmRows];
+    float jx[kAsmRows];
+    const auto fetch = [&](uint32_t e) {  // rows e .. e + kAsmRows - 1 of the list, those before `last`
+        if (((e - first) & 63u) == 0u) ids = r.rows_of[b + min(e + (uint32_t)lane, n - 1)];
+#pragma unroll
+        for (int u = 0; u < kAsmRows; ++u) {
+            const uint32_t row = (uint32_t)__builtin_amdgcn_readlane((int)ids, (int)((e - first + u) & 63u));
+            const bool in = e + u < last && lane < 48;
+            vn[u] = in ? r.node8[8ull * row + q] : kNone;
+            jx[u] = in ? r.j48[48ull * row + lane] : 0.0f;
+        }
+    };
+    static_assert(64 % kAsmRows == 0, "a group of rows lies in one chunk of row numbers");
+    if (first < last) fetch(first);
+    for (uint32_t e0 = first; e0 < last; e0 += kAsmRows) {
         uint32_t v[kAsmRows];
         float j[kAsmRows];
 #pragma unroll
-        for (int u = 0; u < kAsmRows; ++u) {
-            const bool in = e0 + u < n && lane < 48;
-            const uint32_t row = r.rows_of[b + (e0 + u < n ? e0 + u : n - 1)];
-            v[u] = in ? r.node8[8ull * row + q] : kNone;
-            j[u] = in ? r.j48[48ull * row + lane] : 0.0f;
-        }
+        for (int u = 0; u < kAsmRows; ++u) v[u] = vn[u], j[u] = jx[u];
+        if (e0 + kAsmRows < last) fetch(e0 + kAsmRows);
 #pragma unroll
         for (int u = 0; u < kAsmRows; ++u) {
-            if (e0 + u >= n) break;
+            if (e0 + u >= last) break;
             const bool have = v[u] != kNone;
             const uint32_t node = have ? v[u] & 0xffffffu : i;
             const unsigned long long own = __ballot(have && node == i);
