@@ -326,15 +326,16 @@ __device__ __forceinline__ double rsqrt_newton(double s) {
 
 // The diagonal tile D becomes the inverse X of its Cholesky factor, Dt its
 // transpose.  256 threads, thread (tx, ty) holding rows ty + 16 a and columns tx +
-// 16 b in registers; one column a step, which its owners publish with row j of
-// the inverse under construction: A -= l l^T, X(i) -= l(i) X(j).  The chain of 64
-// dependent steps is what a level of few columns waits for; the steps are
-// rolled loops (all 64 columns unrolled over one wave's registers took 42 us: code
-// that runs once comes at the speed of the instruction fetches).  A pivot that
-// is not positive sets sync[2]; sync[3] keeps the largest squared row norm of
-// an inverse (float bits), a lower bound of the norm of JTJ^-1.
+// 16 b in registers; two columns a step, which their owners publish with rows j
+// and j + 1 of the inverse under construction: A -= l l^T, X(i) -= l(i) X(j).  The
+// chain of 32 dependent steps is what a level of few columns waits for (15 us a
+// tile; one column a step took 21); the steps are rolled loops (all 64 columns
+// unrolled over one wave's registers took 42 us: code that runs once comes at the
+// speed of the instruction fetches).  A pivot that is not positive sets sync[2];
+// sync[3] keeps the largest squared row norm of an inverse (float bits), a lower
+// bound of the norm of JTJ^-1.
 __device__ void factor_tile(double* D, double* __restrict__ Dt, int* __restrict__ sync) {
-    __shared__ double s_col[2][kNB], s_row[2][kNB];
+    __shared__ double s_col[2][2][kNB], s_row[2][2][kNB];
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
     double A[4][4], X[4][4];
 #pragma unroll
@@ -349,39 +350,48 @@ __device__ void factor_tile(double* D, double* __restrict__ Dt, int* __restrict_
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
 #pragma unroll 1
-        for (int jj = 0; jj < 16; ++jj) {
-            const int j = 16 * b + jj;
-            double* col = s_col[jj & 1];
-            double* row = s_row[jj & 1];
-            if (tx == jj) {
+        for (int jj = 0; jj < 16; jj += 2) {
+            const int j = 16 * b + jj, u = (jj >> 1) & 1;
+            if ((tx & ~1) == jj) {
 #pragma unroll
-                for (int a = b; a < 4; ++a) col[ty + 16 * a] = A[a][b];
+                for (int a = b; a < 4; ++a) s_col[u][tx & 1][ty + 16 * a] = A[a][b];
             }
-            if (ty == jj) {
+            if ((ty & ~1) == jj) {
 #pragma unroll
-                for (int k = 0; k <= b; ++k) row[tx + 16 * k] = X[b][k];
+                for (int k = 0; k <= b; ++k) s_row[u][ty & 1][tx + 16 * k] = X[b][k];
             }
             __syncthreads();
-            const double s = col[j];
-            ok = ok && s > 0.0;
-            const double inv = rsqrt_newton(s);
-            double lr[4], lc[4], xr[4];
+            const double* col0 = s_col[u][0];
+            const double* col1 = s_col[u][1];
+            const double sa = col0[j];
+            const double inv0 = rsqrt_newton(sa);
+            const double l10 = col0[j + 1] * inv0;  // L(j + 1, j)
+            const double sb = __builtin_fma(-l10, l10, col1[j + 1]);
+            const double inv1 = rsqrt_newton(sb);
+            ok = ok && sa > 0.0 && sb > 0.0;
+            double lr0[4], lc0[4], lr1[4], lc1[4], xr0[4], xr1[4];
 #pragma unroll
             for (int a = b; a < 4; ++a) {
-                lr[a] = col[ty + 16 * a] * inv;
-                lc[a] = col[tx + 16 * a] * inv;
+                lr0[a] = col0[ty + 16 * a] * inv0;
+                lc0[a] = col0[tx + 16 * a] * inv0;
+                lr1[a] = __builtin_fma(-lr0[a], l10, col1[ty + 16 * a]) * inv1;
+                lc1[a] = __builtin_fma(-lc0[a], l10, col1[tx + 16 * a]) * inv1;
             }
 #pragma unroll
-            for (int k = 0; k <= b; ++k) xr[k] = row[tx + 16 * k] * inv;
+            for (int k = 0; k <= b; ++k) {
+                xr0[k] = s_row[u][0][tx + 16 * k] * inv0;
+                xr1[k] = __builtin_fma(-l10, xr0[k], s_row[u][1][tx + 16 * k]) * inv1;
+            }
 #pragma unroll
             for (int a = b; a < 4; ++a) {
 #pragma unroll
-                for (int k = b; k < 4; ++k) A[a][k] = __builtin_fma(-lr[a], lc[k], A[a][k]);
-                const bool own = a == b && ty == jj, done = a == b && ty < jj;
+                for (int k = b; k < 4; ++k)
+                    A[a][k] = __builtin_fma(-lr1[a], lc1[k], __builtin_fma(-lr0[a], lc0[k], A[a][k]));
+                const bool own0 = a == b && ty == jj, own1 = a == b && ty == jj + 1, done = a == b && ty < jj;
 #pragma unroll
                 for (int k = 0; k <= b; ++k) {
-                    const double v = __builtin_fma(-lr[a], xr[k], X[a][k]);
-                    X[a][k] = own ? xr[k] : (done ? X[a][k] : v);
+                    const double v = __builtin_fma(-lr1[a], xr1[k], __builtin_fma(-lr0[a], xr0[k], X[a][k]));
+                    X[a][k] = own0 ? xr0[k] : (own1 ? xr1[k] : (done ? X[a][k] : v));
                 }
             }
         }
