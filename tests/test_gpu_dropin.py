@@ -348,3 +348,39 @@ def test_integrate_plain_rows(vf, oracle, dim, shift, camera):
     bt[shift:shift + n], bw[shift:shift + n] = t, w
     np.testing.assert_array_equal(gt.download(), bt)
     np.testing.assert_array_equal(gw.download(), bw)
+
+
+@pytest.mark.parametrize("dim,shift", [((4, 1, 1), 0), ((64, 9, 5), 0), ((260, 7, 3), 0), ((62, 9, 5), 0),
+                                       ((64, 9, 5), 1), ((64, 9, 5), 2)])
+@pytest.mark.parametrize("k", [3, 4, 8])
+def test_slots_and_vertices_by_alignment(vf, oracle, dim, shift, k):
+    """Vertices, weights and warp on buffers at and off 16 bytes."""
+    n, G = dim[0] * dim[1] * dim[2], 40
+    rng = np.random.default_rng(n + k)
+    vs = (F(0.01),) * 3
+    size = tuple(F(0.01) * F(d) for d in dim)
+    vb = dev(np.full(3 * n + 16, 7, F))
+    L.call("vf_generate_tsdf_vertices", vb.ptr + 4 * shift, L.f3(vs), L.f3(size), L.i3(dim), None)
+    verts = oracle.generate_vertices(dim, vs, size)
+    want = np.full(3 * n + 16, 7, F)
+    want[shift:shift + 3 * n] = verts.reshape(-1)
+    L.call("vf_device_synchronize")
+    np.testing.assert_array_equal(vb.download(), want)
+    idx = rng.integers(0, G, (n, k)).astype(np.uint32)
+    dist = np.sort(rng.uniform(0, 0.05, (n, k)), axis=1).astype(F)
+    cnt = rng.integers(0, k + 2, n).astype(np.int32)
+    radii = rng.uniform(0.01, 0.05, G).astype(F)
+    T = np.tile(np.eye(4, dtype=F).reshape(16), (G, 1)) + (0.01 * rng.normal(size=(G, 16))).astype(F)
+    off = [np.concatenate([np.zeros(shift, a.dtype), a.reshape(-1), np.zeros(8, a.dtype)]) for a in (idx, dist)]
+    g_idx, g_dist, g_w, g_cnt, g_r = dev(off[0]), dev(off[1]), dev(np.zeros(n * k + 16, F)), dev(cnt), dev(radii)
+    L.call("vf_compute_tsdf_warp_weights", k, g_w.ptr + 4 * shift, g_r.ptr, g_idx.ptr + 4 * shift,
+           g_dist.ptr + 4 * shift, g_cnt.ptr, n, None)
+    w = oracle.warp_weights(k, radii, idx, dist, cnt)
+    L.call("vf_device_synchronize")
+    np.testing.assert_array_equal(g_w.download()[shift:shift + n * k].reshape(n, k), w)
+    g_T = dev(T)
+    L.call("vf_warp_tsdf", k, vb.ptr + 4 * shift, g_T.ptr, g_idx.ptr + 4 * shift, g_w.ptr + 4 * shift, g_cnt.ptr,
+           L.f3(vs), L.f3(size), L.i3(dim), None)
+    L.call("vf_device_synchronize")
+    got = vb.download()[shift:shift + 3 * n].reshape(n, 3)
+    np.testing.assert_array_equal(got, oracle.warp_tsdf(k, verts, T, idx, w, cnt))
