@@ -631,6 +631,12 @@ constexpr uint32_t kScEmpty = 4u;  // no target inside the volume: dropped
 constexpr uint32_t kScKeep = 8u;   // screen off for the volume: kept
 constexpr int kMaxScreenTiles = 64;
 
+// t / n for t < 64 and 1 <= n < 1024 as (t * div_magic(n)) >> 16: exact, as the
+// magic exceeds 2^16 / n by at most 1 and t 2^-16 stays below 1 / n.  The walks
+// over tile ranges divide once per brick, not twice per tile (k_compact: 10.0 us
+// for 13.0 of a 512^3 frame, 6.6 for 8.1 of a 72x60x84 one).
+__device__ __forceinline__ uint32_t div_magic(uint32_t n) { return 65536u / n + 1u; }
+
 // Lanes that select one candidate together (k_select) and that screen one
 // brick together (k_compact).  Measured at 512^3 (prep, compaction and
 // selection together): 39.9 us with one lane per screened brick, 41.1, 44.5
@@ -665,8 +671,10 @@ __device__ uint4 screen_brick(const VolDesc& vd, uint32_t b, uint32_t dbits, con
                               int q) {
     if (!vd.screen) return make_uint4(0u, 0u, 0u, kScKeep);
     if (dbits >= kInfBits) return make_uint4(0u, 0u, 0u, kScPend | kScAll);
-    const uint32_t bd0 = (uint32_t)vd.bdim[0], bd1 = (uint32_t)vd.bdim[1];
-    const int32_t bi[3] = {(int32_t)(b % bd0), (int32_t)((b / bd0) % bd1), (int32_t)(b / (bd0 * bd1))};
+    const uint32_t bq = (uint32_t)(((uint64_t)b * vd.bmag[0]) >> vd.bsh[0]);
+    const uint32_t bz = (uint32_t)(((uint64_t)b * vd.bmag[1]) >> vd.bsh[1]);
+    const int32_t bi[3] = {(int32_t)(b - bq * (uint32_t)vd.bdim[0]), (int32_t)(bq - bz * (uint32_t)vd.bdim[1]),
+                           (int32_t)bz};
     const int32_t bs[3] = {S::BX, S::BY, S::BZ};
     const double D = (double)__uint_as_float(dbits);
     double lo[3], hi[3];  // box of the brick's warped voxel positions (camera frame)
@@ -748,12 +756,14 @@ __device__ uint4 screen_brick(const VolDesc& vd, uint32_t b, uint32_t dbits, con
             if (nx * ny > 40) {
                 md = kInf;
             } else {
+                const uint32_t mx = div_magic((uint32_t)nx);
                 for (int32_t t0 = q; t0 < nx * ny; t0 += 8 * GL) {
                     float v[8];
 #pragma unroll
                     for (int u = 0; u < 8; ++u) {
                         const int32_t t = t0 + u * GL;
-                        v[u] = t < nx * ny ? dmax[base + (uint32_t)((ty0 + t / nx) * (int32_t)pw + tx0 + t % nx)]
+                        const int32_t row = (int32_t)(((uint32_t)t * mx) >> 16);
+                        v[u] = t < nx * ny ? dmax[base + (uint32_t)((ty0 + row) * (int32_t)pw + tx0 + t - row * nx)]
                                            : -kInf;
                     }
 #pragma unroll
@@ -859,14 +869,16 @@ __global__ __launch_bounds__(kPrepThreads) void k_compact(
             cand_info[base + c] = info;
         }
         if (info.w & kScPend) {
-            const uint32_t nx = tile_span(info.x), nxy = nx * tile_span(info.y);
+            const uint32_t nx = tile_span(info.x), ny = tile_span(info.y), nxy = nx * ny;
             const uint32_t nt = nxy * tile_span(info.z);
             if ((info.w & kScAll) || nt > (uint32_t)kMaxScreenTiles) {
                 if (q == 0) vol_mark[v] = tag;
             } else {
                 const uint32_t x0 = info.x & 0xffffu, y0 = info.y & 0xffffu, z0 = info.z & 0xffffu;
+                const uint32_t mxy = div_magic(nxy), mx = div_magic(nx);
                 for (uint32_t t = (uint32_t)q; t < nt; t += kGrpC) {
-                    const uint32_t tz = z0 + t / nxy, ty = y0 + (t % nxy) / nx, tx = x0 + t % nx;
+                    const uint32_t lz = (t * mxy) >> 16, r = (t * mx) >> 16;  // layer; row, counted over layers
+                    const uint32_t tz = z0 + lz, ty = y0 + r - lz * ny, tx = x0 + t - r * nx;
                     tile_mark[vd.tile_base + (tz * (uint32_t)vd.tdim[1] + ty) * (uint32_t)vd.tdim[0] + tx] = tag;
                 }
             }
@@ -969,8 +981,9 @@ __global__ __launch_bounds__(kPrepThreads) void k_select(
                 keep = true;
             } else {
                 const uint32_t x0 = info.x & 0xffffu, y0 = info.y & 0xffffu, z0 = info.z & 0xffffu;
-                const uint32_t nx = tile_span(info.x), nxy = nx * tile_span(info.y);
+                const uint32_t nx = tile_span(info.x), ny = tile_span(info.y), nxy = nx * ny;
                 const uint32_t nt = nxy * tile_span(info.z);
+                const uint32_t mxy = div_magic(nxy), mx = div_magic(nx);
                 static_assert(kMaxScreenTiles <= 8 * kGrp, "eight tiles per lane cover the range");
                 uint32_t m[8];
 #pragma unroll
@@ -978,7 +991,8 @@ __global__ __launch_bounds__(kPrepThreads) void k_select(
                     const uint32_t t = (uint32_t)q + (uint32_t)(u * kGrp);
                     m[u] = 0u;
                     if (t < nt) {
-                        const uint32_t tz = z0 + t / nxy, ty = y0 + (t % nxy) / nx, tx = x0 + t % nx;
+                        const uint32_t lz = (t * mxy) >> 16, row = (t * mx) >> 16;
+                        const uint32_t tz = z0 + lz, ty = y0 + row - lz * ny, tx = x0 + t - row * nx;
                         m[u] = tile_mark[(uint32_t)vd.y + (tz * (uint32_t)vd.w + ty) * (uint32_t)vd.z + tx];
                     }
                 }
