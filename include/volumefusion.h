@@ -535,7 +535,7 @@ int vf_gn_normal_equations(vf_workspace* ws, float* JTJ, float* JTr, const float
  * JTJ once (its value does not change during the Gauss-Newton iterations):
  * by Cholesky, JTJ being symmetric positive definite (sparse, in binary64; a
  * dense binary32 one where JTJ's fill is nearly full or its condition number
- * is 2^40 or more), or, where that finds a non-positive pivot, by the LU
+ * is beyond binary32), or, where that finds a non-positive pivot, by the LU
  * with partial pivoting the reference uses (VF_ERR_SINGULAR on a zero pivot).  The problem's buffers must stay alive
  * and unchanged while it exists. */
 typedef struct vf_gn_solver vf_gn_solver;

@@ -344,7 +344,7 @@ def test_gn_crowded_nodes(vf, oracle):
 @pytest.mark.parametrize("kind", ["nearly_singular", "dense_fill"])
 def test_gn_dense_path_where_it_stays(vf, kind):
     """Problems that keep the dense factorisation: parallel normals and a
-    regularisation weight near zero leave directions that binary64 does not
+    regularisation weight near zero leave directions that binary32 does not
     determine; points bound to random nodes couple every part of the graph, so
     that the fill is dense (2.7M tile updates of 64^3).  The dense path's
     residuals are the binary32 ones, so its first energy has the bits of the
@@ -352,7 +352,7 @@ def test_gn_dense_path_where_it_stays(vf, kind):
     import dataclasses
     if kind == "nearly_singular":
         p = scenes.gn_problem(6, G=200, M=6000)
-        p = dataclasses.replace(p, wR=1e-8, dnormals=np.tile(np.array([0, 0, 1], F), (p.dnormals.shape[0], 1)))
+        p = dataclasses.replace(p, wR=1e-4, dnormals=np.tile(np.array([0, 0, 1], F), (p.dnormals.shape[0], 1)))
     else:
         G, M = 2700, 7000
         p = scenes.gn_problem(6, G=G, M=M, K=6)

@@ -1143,14 +1143,14 @@ int sparse_factor(SparseChol* s, const GnRowLists& r, int* good, hipStream_t str
     VF_HIP(hipStreamSynchronize(stream));
     float f[2];
     memcpy(f, h + 1, sizeof(f));
-    // Up to a condition number of 2^40 (a lower bound: the largest diagonal entry
-    // times the inverse's norm bound) binary64 leaves 13 bits in the worst
-    // direction.  From 2^24 on a binary32 factor leaves none there: on 24 graphs
-    // of 4096 nodes, eight of them with a node that hardly anything regularises,
-    // the transforms were off by 1e-4 to 0.15 with it and by 1e-7 to 5e-4 here.
-    // Beyond, JTJ is singular in binary64 as well and the dense path's pivoted
-    // solve decides.
-    *good = h[0] == 0 && f[0] * f[1] < 0x1p40f;
+    // From a condition number of 2^26 on (a lower bound: the largest diagonal
+    // entry times the inverse's norm bound) the rounding of a binary32 JTJ
+    // changes the solution by its own size (a node that no other node
+    // regularises against, on a nearly spherical patch: measured 1.5e8 to
+    // 1e9, against at most 6e7 otherwise, on 36 graphs of 4096 nodes).  The
+    // reference's result there is that of its pivoted binary32 solve; such a
+    // problem keeps the dense path.
+    *good = h[0] == 0 && f[0] * f[1] < 0x1p26f;
     return VF_OK;
 }
 
