@@ -968,8 +968,8 @@ int vf_warp_points(vf_workspace* ws, int k, int blend, vf_float3* warped, const 
     // may not grow the workspace, and the device may be full
     if (lists && workspace_scratch_size(ws) < want) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        VF_HIP(hipStreamIsCapturing((hipStream_t)stream, &cap));
-        lists = cap == hipStreamCaptureStatusNone;
+        lists = hipStreamIsCapturing((hipStream_t)stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+        if (!lists) (void)hipGetLastError();
     }
     st = workspace_scratch(ws, lists ? want : need, &mem, (hipStream_t)stream);
     if (st == VF_ERR_OUT_OF_MEMORY && lists) {
